@@ -168,23 +168,24 @@ PrefillLayout prefill_layout(void* ws, int M, int k, const ftmoe_bank* bank, con
   Carver c{static_cast<uint8_t*>(ws)};
   const int numel = M * k;
   const int H = bank->hidden, I = bank->inter;
-  ftmoe_align_sizes(numel, bank->num_rows, ftmoe::prefill_block_size(bank->format), &L.max_padded, &L.max_blocks);
+  ftmoe_align_sizes(numel, bank->num_rows, ftmoe::prefill_block_size(bank->format, M, k, bank->num_rows, H, I),
+                    &L.max_padded, &L.max_blocks);
   L.sorted = c.take<int32_t>(L.max_padded);
   L.expert_ids = c.take<int32_t>(L.max_blocks);
   L.ntpp = c.take<int32_t>(1);
   L.cum = c.take<int32_t>(bank->num_rows + 2);
   L.gcount = c.take<int32_t>(ftmoe::align_gcount_ints(numel, bank->num_rows));
   const bool quant = bank->format != FTMOE_FMT_BF16;
-  const size_t sc = 4;  // float scale (FP8) or e8m0 code in 32 bits (MXFP4)
+  const size_t sc = bank->format == FTMOE_FMT_FP8_B128 ? 4 : 1;  // float scale (FP8) or e8m0 code (MXFP4)
   const size_t rows = static_cast<size_t>(numel) + (shared ? M : 0);
   if (quant) {
     L.xq = c.take<uint8_t>(static_cast<size_t>(M) * H);
-    L.xs = c.take<uint8_t>(static_cast<size_t>(M) * (H / 128) * sc);
+    L.xs = c.take<uint8_t>(static_cast<size_t>(M) * ftmoe::act_scale_stride(H) * sc);
   }
   if (quant) {  // the gate/up GEMM writes the quantised activations directly
     L.act = nullptr;
     L.actq = c.take<uint8_t>(rows * I);
-    L.as = c.take<uint8_t>(rows * (I / 128) * sc);
+    L.as = c.take<uint8_t>(rows * ftmoe::act_scale_stride(I) * sc);
   } else {
     L.act = c.take<uint16_t>(rows * I);
   }
@@ -431,8 +432,8 @@ int ftmoe_act_quant_fp8(const void* x, int rows, int K, int mode, void* q, void*
   if (rows < 0 || K <= 0 || K % 128 || (mode != 0 && mode != 1))
     return fail(FTMOE_ERR_UNSUPPORTED, "act_quant_fp8: rows=%d K=%d mode=%d", rows, K, mode);
   if (rows == 0) return FTMOE_OK;
-  return check_hip(ftmoe::launch_act_quant(mode, static_cast<const uint16_t*>(x), rows, K, static_cast<uint8_t*>(q),
-                                           scales, stream),
+  return check_hip(ftmoe::launch_act_quant(mode, static_cast<const uint16_t*>(x), rows, K, K / 128,
+                                           static_cast<uint8_t*>(q), scales, stream),
                    "act_quant_fp8 launch");
 }
 
@@ -683,7 +684,8 @@ int ftmoe_experts_prefill(const void* x, int M, int top_k, const float* topk_w, 
   if (M < 0 || top_k <= 0) return fail(FTMOE_ERR_INVALID, "experts_prefill: M=%d top_k=%d", M, top_k);
   if (M == 0) return FTMOE_OK;  // an empty batch: nothing to compute, no pointer is read
   if (!x || !topk_w || !topk_ids || !y) return fail(FTMOE_ERR_INVALID, "experts_prefill: NULL pointer");
-  if (bank->num_rows > 1023) return fail(FTMOE_ERR_UNSUPPORTED, "experts_prefill: num_rows %d > 1023", bank->num_rows);
+  if (bank->num_rows > ftmoe::kPrefillMaxRows)
+    return fail(FTMOE_ERR_UNSUPPORTED, "experts_prefill: num_rows %d > %d", bank->num_rows, ftmoe::kPrefillMaxRows);
   if (activation < FTMOE_ACT_SILU || activation > FTMOE_ACT_GELU_TANH)
     return fail(FTMOE_ERR_UNSUPPORTED, "experts_prefill: activation %d", activation);
   rc = check_limit(bank, shared, activation, "experts_prefill");
@@ -706,7 +708,7 @@ int ftmoe_experts_prefill(const void* x, int M, int top_k, const float* topk_w, 
   al.ids = topk_ids;
   al.numel = numel;
   al.num_experts = bank->num_rows;
-  const int bm = ftmoe::prefill_block_size(bank->format);
+  const int bm = ftmoe::prefill_block_size(fmt, M, top_k, bank->num_rows, H, I);
   al.block_size = bm;
   al.sorted_ids = L.sorted;
   al.max_padded = L.max_padded;
@@ -720,9 +722,9 @@ int ftmoe_experts_prefill(const void* x, int M, int top_k, const float* topk_w, 
   g_timer.mark();
 
   const uint16_t* xb = static_cast<const uint16_t*>(x);
-  const int qmode = fmt == FTMOE_FMT_MXFP4 ? 2 : 0;
+  const int qmode = fmt == FTMOE_FMT_MXFP4 ? 1 : 0;
   if (fmt != FTMOE_FMT_BF16) {
-    rc = check_hip(ftmoe::launch_act_quant(qmode, xb, M, H, L.xq, L.xs, stream), "experts_prefill x quant");
+    rc = check_hip(ftmoe::launch_act_quant(qmode, xb, M, H, ftmoe::act_scale_stride(H), L.xq, L.xs, stream), "experts_prefill x quant");
     if (rc) return rc;
   }
   g_timer.mark();
@@ -734,6 +736,8 @@ int ftmoe_experts_prefill(const void* x, int M, int top_k, const float* topk_w, 
   g.numel = numel;
   g.M = M;
   g.k = top_k;
+  g.k_magic = top_k == 1 ? 0u : static_cast<uint32_t>(((uint64_t{1} << 32) + top_k - 1) / top_k);
+  g.block = bm;
   g.max_blocks = L.max_blocks;
   g.shared_blocks = shared ? (M + bm - 1) / bm : 0;
   g.w = {nullptr, nullptr};

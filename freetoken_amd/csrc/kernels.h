@@ -122,7 +122,7 @@ hipError_t launch_route_shared(const RouteArgs& r, const AlignArgs& al, int fmt_
 struct PrefillGemmArgs {
   // rows of the activation operand
   const uint8_t* xq;        // fp8 [rows, K] (FP8 / MXFP4) or bf16 [rows, K] (BF16)
-  const void* xs;           // float [rows, K/128] (FP8) or uint32 e8m0 codes [rows, K/128] (MXFP4)
+  const void* xs;           // float (FP8) or e8m0 byte codes (MXFP4) [rows, act_scale_stride(K)]
   int x_token_rows;         // 1: gate_up (row = token = route / k, shared row = token)
                             // 0: down    (row = route, shared row = M*k + token)
   const int32_t* sorted;    // [max_padded] route indices per BM block, sentinel numel
@@ -131,6 +131,8 @@ struct PrefillGemmArgs {
   int num_experts;          // bank rows taking part
   int numel;                // M * k
   int M, k;
+  uint32_t k_magic;         // ceil(2^32 / k), 0 for k = 1: r / k = umulhi(r, k_magic) for r < 2^26
+  int block;                // routes per M block (BM)
   int max_blocks;           // routed M blocks of the grid
   int shared_blocks;        // ceil(M / BM) if a shared expert is present, else 0
   int ntiles;               // N tiles
@@ -142,7 +144,7 @@ struct PrefillGemmArgs {
   // outputs
   uint16_t* out;            // gate_up (bf16): act [numel + M, inter]; down: ic3 [numel, N]
   uint8_t* act_q;           // gate_up (FP8, MXFP4): e4m3 act [numel + M, inter] ...
-  void* act_s;              // ... and its scales per 128 (float, or uint32 e8m0 codes)
+  void* act_s;              // ... and its scales per 128 (float, or e8m0 byte codes), rows of act_scale_stride(inter)
   uint16_t* sh_out;         // down: shared out [M, N]
   const float* topk_w;      // [numel] (down)
   int act_kind;
@@ -150,11 +152,36 @@ struct PrefillGemmArgs {
   float sh_act_limit;       // ... of the shared expert
 };
 
-// Routes per M block of the prefill GEMMs (the align block size): the
-// quantised kernels tile 256 routes, the bf16 kernel 128.
-inline int prefill_block_size(int fmt) { return fmt == FMT_BF16 ? 128 : 256; }
+constexpr int kPrefillMaxRows = 1023;  // bank rows of a prefill call
 
-hipError_t launch_act_quant(int mode, const uint16_t* x, int rows, int K, uint8_t* q, void* scales,
+// Routes per M block of the prefill GEMMs (the align block size).  bf16: 128.
+// Quantised formats: 256, or by the mean number of routes per expert r = M k /
+// rows 64 (r <= 48) or 128 (r <= 120): a tile of 256 is then mostly padding.
+// Measured (us, blocks of 64 / 128 / 256): FP8 H 2048, I 768, 128 experts,
+// top-8, r = 31 165 / 172 / 206, r = 69 214 / 189 / 223, r = 112 252 / 223 /
+// 239, r = 137 287 / 263 / 243; MXFP4 of that shape r = 31 118 / 130 / 179, r =
+// 112 201 / 176 / 202, r = 137 234 / 218 / 207; MXFP4 H 5120, I 1536, 160
+// experts, r = 35 502 / 504 / 736, r = 75 713 / 638 / 790.  Uneven routings move
+// the upper line outwards (FP8 H 7168, I 2048, 256 experts, r = 125 3512 / 2971
+// / 3303), but at r = 137 an even one is already 8% slower at 128.
+// The MXFP4 tiles of 256 hold two groups of scales, which costs their copies'
+// overlap across tiles when K / 128 leaves a remainder of 1 by four, and up to
+// 511 experts in LDS: 128 takes those calls.
+inline int prefill_block_size(int fmt, int M, int k, int rows, int H, int I) {
+  if (fmt == FMT_BF16) return 128;
+  const long long routes = static_cast<long long>(M) * k;
+  if (routes <= 48ll * rows) return 64;
+  if (routes <= 120ll * rows) return 128;
+  if (fmt == FMT_MXFP4 && (rows > 511 || H / 128 % 4 == 1 || I / 128 % 4 == 1)) return 128;
+  return 256;
+}
+
+// Scales per row of the prefill's quantised activations: one per 128 values,
+// padded to whole groups of four (the GEMMs copy them four at a time).
+__host__ __device__ constexpr int act_scale_stride(int K) { return (K / 128 + 3) / 4 * 4; }
+
+// mode 0: float32 scales, 1: e8m0 codes (bytes); sstride: scales per row
+hipError_t launch_act_quant(int mode, const uint16_t* x, int rows, int K, int sstride, uint8_t* q, void* scales,
                             hipStream_t stream);
 hipError_t launch_prefill_gemm(int fmt, int gate_up, const PrefillGemmArgs& a, hipStream_t stream);
 

@@ -62,13 +62,13 @@ __device__ __forceinline__ float row16_max_f32(float v) {
 // in flight together; x is read once (nontemporal).
 template <int MODE>
 __global__ void __launch_bounds__(256) act_quant_kernel(const uint16_t* __restrict__ x, int rows, int K,
-                                                        uint8_t* __restrict__ q, void* __restrict__ scales) {
+                                                        uint8_t* __restrict__ q, void* __restrict__ scales,
+                                                        int sstride) {
   const int lane = lane_id();
   const int row = blockIdx.x * 4 + threadIdx.x / kWave;
   if (row >= rows) return;
   const u32x4* xr = reinterpret_cast<const u32x4*>(x + static_cast<size_t>(row) * K);
   uint2* qr = reinterpret_cast<uint2*>(q + static_cast<size_t>(row) * K);
-  const int ng = K / 128;
   const int nv = K / 8;                  // 16-byte pieces of the row
   const int nload = (nv + kWave - 1) / kWave;
   constexpr int kAhead = 8;
@@ -108,10 +108,9 @@ __global__ void __launch_bounds__(256) act_quant_kernel(const uint16_t* __restri
       }
       qr[p] = uint2{pk[0], pk[1]};
       if ((lane & 15) == 0) {
-        const size_t at = static_cast<size_t>(row) * ng + gi;
+        const size_t at = static_cast<size_t>(row) * sstride + gi;
         if (MODE == 0) static_cast<float*>(scales)[at] = sc;
-        else if (MODE == 1) static_cast<uint8_t*>(scales)[at] = static_cast<uint8_t>(sc);
-        else static_cast<uint32_t*>(scales)[at] = static_cast<uint32_t>(sc);
+        else static_cast<uint8_t*>(scales)[at] = static_cast<uint8_t>(sc);
       }
     }
   }
@@ -449,18 +448,26 @@ __global__ void __launch_bounds__(kPThreads) prefill_gemm_kernel(PrefillGemmArgs
 }
 
 // ----------------------------------------------------------------------------
-// Quantised grouped GEMM (FP8, MXFP4) on direct-to-LDS copies
+// Grouped GEMM on direct-to-LDS copies (FP8, MXFP4, bf16)
 //
-// A workgroup of 8 waves computes 256 weight rows x 256 routes (kQBM).  Wave w
-// is row group rg = w/2 (64 weight rows: four 16-row MFMA tiles) and column
-// half ch = w%2 (128 routes: eight 16-column tiles); two waves share each SIMD,
-// so one wave's MFMAs run while the other waits on LDS, folds scales or sits at
-// the barrier.  Every operand of a 128-deep K step -- weight rows, activation
-// tile, weight scales, activation scales -- is copied global -> LDS by the
-// LDS-DMA form of the global loads (no register staging) into a ring of
-// kStages stages: the copies of the next kStages-1 steps are in flight while a
-// step computes.  Waits are explicit (vmcnt of one step's copies) and the
-// barrier is a bare s_barrier, so a barrier never drains copies in flight.
+// A workgroup of 8 waves computes 256 weight rows x BM routes.  Wave w is row
+// group rg = w/2 (64 weight rows: four 16-row MFMA tiles) and column half
+// ch = w%2 (BM/2 routes: BM/32 16-column tiles); two waves share each SIMD, so
+// one wave's MFMAs run while the other waits on LDS, folds scales or sits at
+// the barrier.  Every operand of a K step -- weight rows, activation tile,
+// weight scales, activation scales -- is copied global -> LDS by the LDS-DMA
+// form of the global loads (no register staging) into a ring of kStages
+// stages: the copies of the next kStages-1 steps are in flight while a step
+// computes.  Waits are explicit (vmcnt of whole steps' copies) and the barrier
+// is a bare s_barrier, so a barrier never drains copies in flight.  A K step
+// is one 128-byte line of every row: 128 values of the quantised formats (64
+// bytes of MXFP4 weights), 64 of bf16.
+//
+// Routes per tile (BM, prefill_block_size): 256 where the experts have that
+// many routes; 128 and 64 for shorter batches, where a tile of 256 is mostly
+// padding columns whose MFMAs, LDS reads and scale folds cost as much as real
+// ones, while the bound is the stream of the weights.  The smaller tiles'
+// stages leave room for a deeper ring.
 //
 // LDS lines (a weight row or an activation column of one K step: 128 bytes,
 // 64 for MXFP4 weights) are stored as 16-byte chunks XOR-swizzled by the line
@@ -481,7 +488,6 @@ __global__ void __launch_bounds__(kPThreads) prefill_gemm_kernel(PrefillGemmArgs
 // its N tiles: the workgroups an XCD runs at once read several weight tiles and
 // share the activations of a few M blocks.
 // ----------------------------------------------------------------------------
-constexpr int kQBM = 256;     // routes per tile (align block size of the quantised formats)
 constexpr int kQRows = 256;   // weight rows per workgroup
 constexpr int kQThreads = 512;
 constexpr int kXcds = 8;
@@ -489,29 +495,46 @@ constexpr int kXcds = 8;
 // Measured on C5 (interleaved A/B, ms): FP8 gate_up 4 -> 2.23-2.24, 8 -> 2.19-2.20,
 // 16 -> 2.22, 2 -> 2.32; FP8 down 4 -> 1.25-1.26, 2 -> 1.20, 1 -> 1.22; MXFP4
 // gate_up 4 -> 1.79 (2 and 8 slower by 4-7%); MXFP4 down 4 -> 1.04-1.06, 2 ->
-// 1.02-1.04, 8 -> 1.09-1.10.
+// 1.02-1.04, 8 -> 1.09-1.10.  Tiles of 128 and 64 routes take twice and four
+// times as many (the same routes).
 constexpr int kQChunkSel[2][2] = {{8, 2}, {4, 2}};
-template <int FMT, int GATE_UP>
+template <int FMT, int GATE_UP, int BM>
 constexpr int q_chunk() {
-  return kQChunkSel[FMT == FMT_FP8 ? 0 : 1][GATE_UP ? 0 : 1];
+  return kQChunkSel[FMT == FMT_MXFP4 ? 1 : 0][GATE_UP ? 0 : 1] * (256 / BM);
 }
-constexpr int kFoldLag = 3;  // FP8: MFMAs between an MFMA and the fold of its result
+constexpr int kFoldLag = 2;  // FP8: MFMAs between an MFMA and the fold of its result (3: 1% slower)
 
-template <int FMT>
+template <int FMT, int BM>
 struct QLds {
-  static constexpr int kStages = FMT == FMT_FP8 ? 2 : 3;
-  static constexpr int kALine = FMT == FMT_FP8 ? 128 : 64;   // weight bytes per row per K step
+  // as many stages as fit 160 KB beside the scales and the tile's lists
+  static constexpr int kStages = FMT == FMT_MXFP4 ? (BM == 256 ? 3 : BM == 128 ? 4 : 5) : (BM == 256 ? 2 : 3);
+  static constexpr bool kQuant = FMT != FMT_BF16;
+  static constexpr int kStepK = kQuant ? 128 : 64;            // K values per step
+  static constexpr int kALine = FMT == FMT_MXFP4 ? 64 : 128;  // weight bytes per row per K step
   static constexpr int kA = kQRows * kALine;
-  static constexpr int kAS = FMT == FMT_FP8 ? 4 * 16 : kQRows * 4;  // fp8: 4 floats per row group; mxfp4: 4 codes per row
-  static constexpr int kB = kQBM * 128;
-  static constexpr int kBS = kQBM * 4;
-  static constexpr int kOffAS = kA, kOffB = kA + kAS, kOffBS = kA + kAS + kB;
-  static constexpr int kStage = kA + kAS + kB + kBS;
-  static constexpr int kTotal = kStages * kStage;
+  static constexpr int kB = BM * 128;
+  static constexpr int kStage = kA + kB;
+  static constexpr int kRing = kStages * kStage;
   static constexpr int kACopies = kA / 1024 / 8;   // 1 KB copies per wave per step
   static constexpr int kBCopies = kB / 1024 / 8;
-  // LDS-DMA instructions each wave issues per K step (uniform over waves)
-  static constexpr int kDmaPerStep = kACopies + kBCopies + 1;
+  // LDS-DMA instructions each wave issues per K step (uniform over waves; the
+  // scale groups come on top)
+  static constexpr int kDmaPerStep = kACopies + kBCopies;
+  // Scales are copied for four K steps at once, 16 bytes of a row's float32
+  // scales or e8m0 codes per lane (4 bytes of the activations' byte codes): a
+  // copy per step fetched 4 bytes of every row's line, as many lines per step
+  // as the weights and activations together (without any scale copies, timing
+  // only, MXFP4 H 5120, I 1536, 12000 routes over 160 experts took 714 -> 648
+  // us; in groups 658).  A group's buffer is written D steps before its first
+  // step: with three buffers the one written is never in use; with two (what
+  // fits beside 256 routes) it is only where a tile's last group is shorter
+  // than D, and such a tile does not run ahead into the next.
+  static constexpr int kWS = FMT == FMT_FP8 ? 4 * 64 : FMT == FMT_MXFP4 ? kQRows * 16 : 0;
+  static constexpr int kXS = FMT == FMT_FP8 ? BM * 16 : FMT == FMT_MXFP4 ? BM * 4 : 0;
+  static constexpr int kGroup = kWS + kXS;
+  static constexpr int kGroups = BM == 256 ? 2 : 3;
+  // LDS before the expert list
+  static constexpr int kFixed = kRing + kGroups * kGroup;
 };
 
 __device__ __forceinline__ int xcd_major(int b, int n) {
@@ -537,38 +560,6 @@ __device__ __forceinline__ void chunked(int local, int nb, int ntiles, int& m, i
   }
 }
 
-// Workgroup b of the grid -> (expert or shared, M block, N tile).  Only the
-// active workgroups -- routed blocks of the real experts, then the shared
-// expert's blocks -- take part; they are laid out XCD-major over their own
-// count, so every XCD gets the same share.  Returns false for idle ones.
-template <int kQChunk>
-__device__ __forceinline__ bool map_tile_q(const PrefillGemmArgs& a, int b, bool& shared, int& expert, int& mblock,
-                                           int& ntile) {
-  const int routed = (a.cum[a.num_experts] / kQBM) * a.ntiles;
-  const int total = routed + a.shared_blocks * a.ntiles;
-  if (b >= total) return false;
-  const int wg = xcd_major(b, total);
-  if (wg < routed) {
-    int lo = 0, hi = a.num_experts;  // largest e with cum[e]/BM * ntiles <= wg
-    while (hi - lo > 1) {
-      const int mid = (lo + hi) >> 1;
-      if ((a.cum[mid] / kQBM) * a.ntiles <= wg) lo = mid; else hi = mid;
-    }
-    const int b0 = a.cum[lo] / kQBM;
-    const int nb = a.cum[lo + 1] / kQBM - b0;
-    int m;
-    chunked<kQChunk>(wg - b0 * a.ntiles, nb, a.ntiles, m, ntile);
-    shared = false;
-    expert = lo;
-    mblock = b0 + m;
-    return true;
-  }
-  chunked<kQChunk>(wg - routed, a.shared_blocks, a.ntiles, mblock, ntile);
-  shared = true;
-  expert = 0;
-  return true;
-}
-
 // Lane index as an asm result: the compiler can neither hoist nor merge it,
 // so per-tile set-up code recomputes its lane-derived values instead of keeping
 // them live (or spilled) across the K loop.
@@ -583,9 +574,46 @@ struct QTile {
   int expert, mblock, ntile;
 };
 
+// Workgroup b of the grid -> (expert or shared, M block, N tile).  Only the
+// active workgroups -- routed blocks of the real experts, then the shared
+// expert's blocks -- take part; they are laid out XCD-major over their own
+// count, so every XCD gets the same share.  Returns false for idle ones.
+// s_blk (LDS): the first M block of every expert, [num_experts] the routed
+// total.  The owner of a position is found by the whole wave at once (one
+// ballot per 64 experts): a binary search over the regions in global memory
+// was a chain of dependent loads at every tile, each of whose waits drained
+// the copies in flight.
 template <int kQChunk>
-__device__ __forceinline__ bool map_tile_q(const PrefillGemmArgs& a, int b, QTile& t) {
-  return map_tile_q<kQChunk>(a, b, t.shared, t.expert, t.mblock, t.ntile);
+__device__ __forceinline__ bool map_tile_q(const PrefillGemmArgs& a, const int* s_blk, int b, QTile& t) {
+  const int E = a.num_experts;
+  const int routed = __builtin_amdgcn_readfirstlane(s_blk[E]) * a.ntiles;
+  const int total = routed + a.shared_blocks * a.ntiles;
+  if (b >= total) return false;
+  const int wg = xcd_major(b, total);
+  if (wg < routed) {
+    int owner = -1;  // largest e whose first tile is <= wg
+    for (int e0 = 0; e0 < E; e0 += 4 * kWave) {
+      int first[4];  // four reads in flight (entries past the last expert: its neighbours)
+      const int l = fresh_lane();
+#pragma unroll
+      for (int u = 0; u < 4; ++u) first[u] = s_blk[min(e0 + u * kWave + l, E)];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) owner += __popcll(__ballot(e0 + u * kWave + l < E && first[u] * a.ntiles <= wg));
+    }
+    owner = __builtin_amdgcn_readfirstlane(owner);
+    const int b0 = __builtin_amdgcn_readfirstlane(s_blk[owner]);
+    const int nb = __builtin_amdgcn_readfirstlane(s_blk[owner + 1]) - b0;
+    int m;
+    chunked<kQChunk>(wg - b0 * a.ntiles, nb, a.ntiles, m, t.ntile);
+    t.shared = false;
+    t.expert = owner;
+    t.mblock = b0 + m;
+    return true;
+  }
+  chunked<kQChunk>(wg - routed, a.shared_blocks, a.ntiles, t.mblock, t.ntile);
+  t.shared = true;
+  t.expert = 0;
+  return true;
 }
 
 // s_barrier without the memory fence of __syncthreads (which would wait for
@@ -613,96 +641,84 @@ __device__ __forceinline__ void lds_buf4(__amdgpu_buffer_rsrc_t r, uint8_t* dst,
 
 // Chunk swizzles of the LDS lines, chosen by measurement (rocprofv3
 // SQ_LDS_BANK_CONFLICT over ds_read_b128 patterns on gfx950): for 128-byte
-// lines read as chunk pairs (2g, 2g+1) -- the FP8 operands -- position
+// lines read as chunk pairs (2g, 2g+1) -- the FP8 and bf16 operands -- position
 // c ^ swz_pair(line) is conflict-free while c ^ (line & 7) is not; for lines
 // read as chunks (g, 4+g) -- the MXFP4 activations -- c ^ (line & 7) is
 // conflict-free; for 64-byte lines read as chunk g -- the MXFP4 weights --
 // c ^ ((line >> 1) & 3) is.
 __device__ __forceinline__ int swz_pair(int line) { return ((line & 3) << 1) | ((line >> 2) & 1); }
 template <int FMT>
-__device__ __forceinline__ int swz_b(int line) { return FMT == FMT_FP8 ? swz_pair(line) : (line & 7); }
+__device__ __forceinline__ int swz_b(int line) { return FMT == FMT_MXFP4 ? (line & 7) : swz_pair(line); }
 __device__ __forceinline__ int swz64(int line) { return (line >> 1) & 3; }
 
 // Empty asm that keeps the value's update at this point of the instruction
 // stream (no code is emitted).
 __device__ __forceinline__ void pin(f32x4& v) { asm volatile("" : "+v"(v)); }
 
-template <int FMT, int GATE_UP>
-__global__ void __launch_bounds__(kQThreads) prefill_qgemm_kernel(PrefillGemmArgs a) {
-  using L = QLds<FMT>;
-  constexpr int S = L::kStages;
-  constexpr int D = S - 1;  // prefetch distance in K steps
-  extern __shared__ __attribute__((aligned(16))) uint8_t q_lds[];
-  __shared__ int s_row[2][kQBM];    // per tile parity: activation row of each route column (-1: padding)
-  __shared__ int s_route[2][kQBM];  // per tile parity: route of each column (-1: padding)
-  __shared__ float s_amax[GATE_UP ? 4 * kQBM : 1];  // gate_up epilogue: [row group][column] amax
-  __shared__ float s_wt[GATE_UP ? 1 : 2][kQBM];      // down: per tile parity, router weight of each column
+__device__ __forceinline__ uint64_t uniform_u64(uint64_t v) { return readlane_u64(v, 0); }
 
-  int v = blockIdx.x;
-  QTile cur;
-  constexpr int kChunk = q_chunk<FMT, GATE_UP>();
-  if (!map_tile_q<kChunk>(a, v, cur)) return;
+template <int FMT, int GATE_UP, int BM>
+__global__ void __launch_bounds__(kQThreads) prefill_qgemm_kernel(PrefillGemmArgs a) {
+  using L = QLds<FMT, BM>;
+  constexpr int S = L::kStages;
+  constexpr int D = S - 1;       // prefetch distance in K steps
+  constexpr int NCT = BM / 32;   // 16-column tiles per wave
+  constexpr bool kQuant = L::kQuant;
+  // ring of stages, scale groups, then the first M block of every expert ([num_experts + 1])
+  extern __shared__ __attribute__((aligned(16))) uint8_t q_lds[];
+  int* const s_blk = reinterpret_cast<int*>(q_lds + L::kFixed);
+  // per tile parity: each route column's route (shared tiles: token); padding
+  // columns hold a value at or past the tile's limit (col_limit)
+  __shared__ int s_route[2][BM];
+  __shared__ float s_wt[GATE_UP ? 1 : 2][BM];  // down: per tile parity, router weight of each column
 
   const int tid = threadIdx.x;
   const int lane = lane_id();
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int rg = wave >> 1, ch = wave & 1;
   const int r16 = lane & 15, g = lane >> 4;
-  const int K = a.K, nkb = K / 128;
-  const uint32_t rb = FMT == FMT_FP8 ? static_cast<uint32_t>(K) : static_cast<uint32_t>(K) / 2;
+  const int K = a.K, nkb = K / L::kStepK, nsc = K / 128;
+  const int ngrp = (nkb + 3) / 4;  // scale groups of a tile
+  const uint32_t xsb = FMT == FMT_FP8 ? act_scale_stride(K) * 4u : 1u * act_scale_stride(K);  // bytes of a row's scales
+  // bytes of a weight row and of an activation row
+  const uint32_t rb = FMT == FMT_BF16 ? 2u * K : FMT == FMT_FP8 ? 1u * K : static_cast<uint32_t>(K) / 2;
+  const uint32_t xb = FMT == FMT_BF16 ? 2u * K : 1u * K;
 
-  // column tid of tile t from its align entry `raw` (routed tiles) and, for
-  // the down GEMM, the route's router weight wraw (loaded with raw, well
-  // before this call, so its latency stays off the epilogue)
-  auto put_rows = [&](const QTile& t, int raw, float wraw, int b) {
-    const int tid = wave * kWave + fresh_lane();
-    int row = -1, route = -1;
-    if (t.shared) {
-      const int tk = t.mblock * kQBM + tid;
-      if (tk < a.M) {
-        route = tk;
-        row = a.x_token_rows ? tk : a.numel + tk;
-      }
-    } else if (raw < a.numel) {
-      route = raw;
-      row = a.x_token_rows ? raw / a.k : raw;
-    }
-    s_row[b][tid] = row;
-    s_route[b][tid] = route;
-    if constexpr (!GATE_UP) s_wt[b][tid] = t.shared ? 1.0f : wraw;
-  };
-  auto raw_of = [&](const QTile& t) -> int { return t.shared ? 0 : a.sorted[t.mblock * kQBM + tid]; };
-  auto wt_of = [&](const QTile& t, int raw) -> float {
-    return (GATE_UP || t.shared || raw >= a.numel) ? 1.0f : a.topk_w[raw];
-  };
+  for (int e = tid; e <= a.num_experts; e += kQThreads) s_blk[e] = a.cum[e] / BM;
+  __syncthreads();
+  int v = blockIdx.x;
+  QTile cur;
+  constexpr int kChunk = q_chunk<FMT, GATE_UP, BM>();
+  if (!map_tile_q<kChunk>(a, s_blk, v, cur)) return;
+
   auto n0_of = [&](const QTile& t) -> int { return GATE_UP ? t.ntile * (kQRows / 2) : t.ntile * kQRows; };
   // first weight row of tile j of row group q, relative to the tile's first row n0
   auto trow_rel = [&](int q, int j) -> int {
     if (GATE_UP) return (j < 2 ? 0 : a.inter) + 32 * q + 16 * (j & 1);
     return 64 * q + 16 * j;
   };
+  // columns of tile t with s_route at or past this are padding
+  auto col_limit = [&](const QTile& t) -> int { return t.shared ? a.M : a.numel; };
 
   // ---- sources of the copies: buffer descriptors + 32-bit lane offsets of K
   // step 0 (step kb adds kb * step bytes as the scalar offset).  Weight rows,
   // weight scales and activation rows past their range (the last down tile's
   // rows past N, padding route columns) read zeros without memory traffic.
   const int xrows = a.x_token_rows ? a.M : a.numel + a.M;
-  const __amdgpu_buffer_rsrc_t rsrc_x = make_rsrc(a.xq, static_cast<uint32_t>(xrows) * K);
-  __amdgpu_buffer_rsrc_t rsrc_w;
-  // scales: the activation scales' descriptor is the kernel's; the weight
-  // scales' is set per tile for every wave (waves 4-7 never use it), so that
-  // both stay wave-uniform values in scalar registers (a descriptor assigned
-  // under a per-wave condition was kept in vector registers and every copy
-  // became a loop over its distinct values)
-  const __amdgpu_buffer_rsrc_t rsrc_xs = make_rsrc(a.xs, static_cast<uint32_t>(xrows) * nkb * 4);
-  __amdgpu_buffer_rsrc_t rsrc_ws = rsrc_xs;
+  const __amdgpu_buffer_rsrc_t rsrc_x = make_rsrc(a.xq, static_cast<uint32_t>(xrows) * xb);
+  // (the weights' and scales' ranges are kept as wave-uniform integers: as
+  // descriptors carried from tile to tile they were held in vector registers,
+  // and every copy ran as a loop over their distinct values)
+  uint64_t wbase = 0;
+  uint32_t wrange = 0;
+  const __amdgpu_buffer_rsrc_t rsrc_wt = make_rsrc(a.topk_w, static_cast<uint32_t>(a.numel) * 4);
   // weights: copy c of wave w fills LDS rows of 1 KB block i = w*kACopies + c
   uint32_t avoff[L::kACopies];
 #pragma unroll
   for (int c = 0; c < L::kACopies; ++c) {
     const int i = wave * L::kACopies + c;
     int R, q;
-    if constexpr (FMT == FMT_FP8) {
+    if constexpr (FMT != FMT_MXFP4) {
       R = 8 * i + (lane >> 3);
       q = (lane & 7) ^ swz_pair(R);
     } else {
@@ -712,119 +728,145 @@ __global__ void __launch_bounds__(kQThreads) prefill_qgemm_kernel(PrefillGemmArg
     avoff[c] = static_cast<uint32_t>(trow_rel(R >> 6, (R >> 4) & 3) + (R & 15)) * rb + q * 16;
   }
   // scales: waves 0-3 copy their row group's weight scales (offsets fixed
-  // relative to the tile), waves 4-7 64 activation-scale columns each
+  // relative to the tile), the next BM/64 waves 64 activation-scale columns each
+  // (sbase, srange: the array this wave copies from; slanes lanes take part)
+  const int slanes = wave < 4 ? (FMT == FMT_FP8 ? 4 : kWave) : wave < 4 + BM / 64 ? kWave : 0;
+  const int sdst = __builtin_amdgcn_readfirstlane(wave < 4 ? wave * (L::kWS / 4) : L::kWS + (wave - 4) * (L::kXS / (BM / 64)));
+  uint64_t sbase = reinterpret_cast<uint64_t>(a.xs);
+  uint32_t srange = kQuant ? static_cast<uint32_t>(xrows) * xsb : 0u;
   uint32_t svoff = 0;
-  if (wave < 4) {
-    if constexpr (FMT == FMT_FP8) svoff = static_cast<uint32_t>(trow_rel(wave, lane & 3) / 128) * nkb * 4;
+  if (kQuant && wave < 4) {
+    if constexpr (FMT == FMT_FP8) svoff = static_cast<uint32_t>(trow_rel(wave, lane & 3) / 128) * nsc * 4;
     else svoff = static_cast<uint32_t>(trow_rel(wave, lane >> 4) + (lane & 15)) * (K / 32);
   }
-  uint8_t* const sdst_base = q_lds + (wave < 4 ? (FMT == FMT_FP8 ? L::kOffAS + wave * 16 : L::kOffAS + wave * 256)
-                                               : L::kOffBS + (wave - 4) * 256);
-  const bool scopy = wave >= 4 || FMT != FMT_FP8 || lane < 4;
   // activations: copy c of wave w fills LDS columns of 1 KB block i = w*kBCopies + c
   uint32_t xvoff[L::kBCopies];
   auto setup = [&](const QTile& t, int b) {
     const BankView bank = t.shared ? a.ws : a.w;
     const int n0 = n0_of(t);
-    rsrc_w = make_rsrc(bank.w + (static_cast<size_t>(t.expert) * a.N + n0) * rb, static_cast<uint32_t>(a.N - n0) * rb);
-    if constexpr (FMT == FMT_FP8)
-      rsrc_ws = make_rsrc(static_cast<const uint8_t*>(bank.s) +
-                              (static_cast<size_t>(t.expert) * (a.N / 128) + n0 / 128) * nkb * 4,
-                          static_cast<uint32_t>((a.N - n0) / 128) * nkb * 4);
-    else
-      rsrc_ws = make_rsrc(static_cast<const uint8_t*>(bank.s) + (static_cast<size_t>(t.expert) * a.N + n0) * (K / 32),
-                          static_cast<uint32_t>(a.N - n0) * (K / 32));
+    wbase = uniform_u64(reinterpret_cast<uint64_t>(bank.w) + (static_cast<uint64_t>(t.expert) * a.N + n0) * rb);
+    wrange = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(a.N - n0) * rb);
+    if (kQuant && wave < 4) {
+      const uint32_t srow = FMT == FMT_FP8 ? static_cast<uint32_t>(nsc) * 4 : static_cast<uint32_t>(K) / 32;
+      const int nrow = FMT == FMT_FP8 ? a.N / 128 : a.N, r0 = FMT == FMT_FP8 ? n0 / 128 : n0;
+      const uint64_t at = reinterpret_cast<uint64_t>(bank.s) + (static_cast<uint64_t>(t.expert) * nrow + r0) * srow;
+      sbase = uniform_u64(at);
+      srange = __builtin_amdgcn_readfirstlane((nrow - r0) * srow);
+    }
+    // activation row of a column: gate_up the token, down the route (the
+    // shared expert's tokens follow the routes)
+    const int lim = col_limit(t);
+    const uint32_t magic = !t.shared && a.x_token_rows ? a.k_magic : 0u;
+    const int add = t.shared && !a.x_token_rows ? a.numel : 0;
+    auto row_of = [&](int r) -> uint32_t { return (magic ? __umulhi(static_cast<uint32_t>(r), magic) : static_cast<uint32_t>(r)) + add; };
     const int ln = fresh_lane();
-    if (wave >= 4) {
-      const int row = s_row[b][64 * (wave - 4) + ln];
-      svoff = row < 0 ? kOutOfRange : static_cast<uint32_t>(row) * nkb * 4;
+    if (kQuant && wave >= 4 && wave < 4 + BM / 64) {
+      const int r = s_route[b][64 * (wave - 4) + ln];
+      svoff = r >= lim ? kOutOfRange : row_of(r) * xsb;
     }
 #pragma unroll
     for (int c = 0; c < L::kBCopies; ++c) {
       const int col = 8 * (wave * L::kBCopies + c) + (ln >> 3);
       const int q = (ln & 7) ^ swz_b<FMT>(col);
-      const int row = s_row[b][col];
-      xvoff[c] = row < 0 ? kOutOfRange : static_cast<uint32_t>(row) * K + q * 16;
+      const int r = s_route[b][col];
+      xvoff[c] = r >= lim ? kOutOfRange : row_of(r) * xb + q * 16;
+    }
+    if (!GATE_UP && !t.shared && wave < BM / 64) {
+      const int r = s_route[b][64 * wave + ln];
+      lds_buf4(rsrc_wt, reinterpret_cast<uint8_t*>(&s_wt[b][64 * wave]),
+               r >= lim ? kOutOfRange : static_cast<uint32_t>(r) * 4, 0);
     }
   };
 
-  // piece q of a K step's copies (weight copies, activation copies, scales)
-  constexpr int kPieces = L::kACopies + L::kBCopies + 1;
+  // piece q of a K step's copies (weight copies, activation copies)
+  constexpr int kPieces = L::kDmaPerStep;
   auto issue_piece = [&](int q, int kb, int stg) {
     uint8_t* st = q_lds + stg * L::kStage;
     if (q < L::kACopies) {
-      lds_buf16(rsrc_w, st + (wave * L::kACopies + q) * 1024, avoff[q], static_cast<uint32_t>(kb) * L::kALine);
-    } else if (q < L::kACopies + L::kBCopies) {
-      const int c = q - L::kACopies;
-      lds_buf16(rsrc_x, st + L::kOffB + (wave * L::kBCopies + c) * 1024, xvoff[c], static_cast<uint32_t>(kb) * 128);
-    } else if (wave < 4) {
-      if (scopy) lds_buf4(rsrc_ws, sdst_base + stg * L::kStage, svoff, static_cast<uint32_t>(kb) * 4);
+      lds_buf16(make_rsrc(reinterpret_cast<const void*>(wbase), wrange), st + (wave * L::kACopies + q) * 1024, avoff[q], static_cast<uint32_t>(kb) * L::kALine);
     } else {
-      lds_buf4(rsrc_xs, sdst_base + stg * L::kStage, svoff, static_cast<uint32_t>(kb) * 4);
+      const int c = q - L::kACopies;
+      lds_buf16(rsrc_x, st + L::kA + (wave * L::kBCopies + c) * 1024, xvoff[c], static_cast<uint32_t>(kb) * 128);
     }
   };
-  auto issue = [&](int kb, int stg) {
-    uint8_t* st = q_lds + stg * L::kStage;
-#pragma unroll
-    for (int c = 0; c < L::kACopies; ++c)
-      lds_buf16(rsrc_w, st + (wave * L::kACopies + c) * 1024, avoff[c], static_cast<uint32_t>(kb) * L::kALine);
-#pragma unroll
-    for (int c = 0; c < L::kBCopies; ++c)
-      lds_buf16(rsrc_x, st + L::kOffB + (wave * L::kBCopies + c) * 1024, xvoff[c], static_cast<uint32_t>(kb) * 128);
-    if (wave < 4) {
-      if (scopy) lds_buf4(rsrc_ws, sdst_base + stg * L::kStage, svoff, static_cast<uint32_t>(kb) * 4);
-    } else {
-      lds_buf4(rsrc_xs, sdst_base + stg * L::kStage, svoff, static_cast<uint32_t>(kb) * 4);
+  // the scales of steps kb .. kb+3 (kb % 4 == 0; past the last step unused
+  // values) into group buffer grp
+  auto scale_group = [&](int grp) { return q_lds + __builtin_amdgcn_readfirstlane(L::kRing + grp * L::kGroup); };
+  auto issue_scales = [&](int kb, int grp) {
+    if constexpr (FMT == FMT_FP8) {
+      // one instruction for both kinds, its descriptor chosen per wave by
+      // scalar selects (with a branch per kind the compiler merged the two
+      // into one copy whose descriptor sat in vector registers, which runs as
+      // a loop over its distinct values)
+      const __amdgpu_buffer_rsrc_t rs = make_rsrc(reinterpret_cast<const void*>(sbase), srange);
+      uint8_t* const gs = scale_group(grp) + sdst;
+      if (lane < slanes) lds_buf16(rs, gs, svoff, static_cast<uint32_t>(kb) * 4);
+    } else if constexpr (FMT == FMT_MXFP4) {
+      uint8_t* const gs = scale_group(grp) + sdst;
+      const __amdgpu_buffer_rsrc_t rs = make_rsrc(reinterpret_cast<const void*>(sbase), srange);
+      if (wave < 4) lds_buf16(rs, gs, svoff, static_cast<uint32_t>(kb) * 4);
+      else if (wave < 4 + BM / 64) lds_buf4(rs, gs, svoff, static_cast<uint32_t>(kb));
     }
+  };
+  auto issue = [&](int kb, int stg, int gb) {
+    if ((kb & 3) == 0) issue_scales(kb, (gb + (kb >> 2)) % L::kGroups);
+#pragma unroll
+    for (int q = 0; q < kPieces; ++q) issue_piece(q, kb, stg);
   };
 
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-  f32x4 acc[4][8];
+  f32x4 acc[4][NCT];
 
-  // One K step from stage stg.  With ikb >= 0 the copies of step ikb into
-  // stage istg are issued two per column tile in the first tiles, between the
+  // K step kb from stage stg, scales from the groups that start at gb.  With
+  // ikb >= 0 the copies of step ikb into stage istg (groups from igb) are issued a few per column tile in the first tiles, between the
   // LDS reads and MFMAs, instead of as one burst before the step (a burst
   // stalls the wave's in-order issue until the memory pipeline takes it:
-  // measured 3% of the FP8 gate_up GEMM; MXFP4, whose 3-stage ring already
-  // spills a few registers, keeps the burst).
-  constexpr bool kSpread = FMT == FMT_FP8;
-  auto compute = [&](int stg, int ikb, int istg) {
+  // measured 3% of the FP8 gate_up GEMM; MXFP4 with 256-route tiles, whose
+  // 3-stage ring already spills a few registers, keeps the burst).
+  constexpr bool kSpread = FMT != FMT_MXFP4 || BM < 256;
+  constexpr int kPer = NCT == 8 ? 2 : (kPieces + NCT - 1) / NCT;  // pieces per column tile
+  auto compute = [&](int kb, int stg, int gb, int ikb, int istg, int igb) {
     const uint8_t* st = q_lds + stg * L::kStage;
+    if (ikb >= 0 && (ikb & 3) == 0) issue_scales(ikb, (igb + (ikb >> 2)) % L::kGroups);
+    const uint8_t* sg = scale_group((gb + (kb >> 2)) % L::kGroups);
+    const int sq = kb & 3;  // step of the group
     i32x8 wf[4];
     int wcode[4];
     float sw[4];
     auto read_w = [&](int j) {
       const int R = 64 * rg + 16 * j + r16;
-      if constexpr (FMT == FMT_FP8) {
+      if constexpr (FMT != FMT_MXFP4) {
         const uint8_t* p = st + R * 128;
         const u32x4 lo = *reinterpret_cast<const u32x4*>(p + (((2 * g) ^ swz_pair(R)) * 16));
         const u32x4 hi = *reinterpret_cast<const u32x4*>(p + (((2 * g + 1) ^ swz_pair(R)) * 16));
         wf[j] = i32x8{(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
-        sw[j] = *reinterpret_cast<const float*>(st + L::kOffAS + rg * 16 + j * 4);
+        if constexpr (FMT == FMT_FP8) sw[j] = *reinterpret_cast<const float*>(sg + rg * 64 + j * 16 + sq * 4);
       } else {
         const u32x4 v4 = *reinterpret_cast<const u32x4*>(st + R * 64 + ((g ^ swz64(R)) * 16));
         wf[j] = i32x8{(int)v4[0], (int)v4[1], (int)v4[2], (int)v4[3], 0, 0, 0, 0};
-        wcode[j] = st[L::kOffAS + R * 4 + g];
+        wcode[j] = sg[R * 16 + sq * 4 + g];
       }
     };
-    // Column tile i reads route column 128ch + 16i + r16.  The chunk swizzle
+    // Column tile i reads route column (BM/2)ch + 16i + r16.  The chunk swizzle
     // depends on the column's low 3 bits (those of r16) only, so every tile's
     // reads are one per-lane base of the step plus a compile-time offset
-    // (2048 B per tile for the codes, 64 B for the scales): no address
+    // (2048 B per tile for the codes, 256 or 64 B for the scales): no address
     // arithmetic per tile.  The f8f6f4 MFMA reads an fp8 lane group g as
     // K = 16g+[0,16) and 64+16g+[0,16), an fp4 lane group as the block
-    // [32g, 32g+32).
-    const int c0 = 128 * ch + r16;
-    const int q_lo = FMT == FMT_FP8 ? (2 * g) ^ swz_b<FMT>(r16) : g ^ swz_b<FMT>(r16);
-    const int q_hi = FMT == FMT_FP8 ? (2 * g + 1) ^ swz_b<FMT>(r16) : (4 + g) ^ swz_b<FMT>(r16);
-    const uint8_t* const x_lo = st + L::kOffB + c0 * 128 + q_lo * 16;
-    const uint8_t* const x_hi = st + L::kOffB + c0 * 128 + q_hi * 16;
-    const uint8_t* const x_sc = st + L::kOffBS + c0 * 4;
+    // [32g, 32g+32); the bf16 MFMAs take chunk 2g of both operands, then
+    // chunk 2g+1.
+    const int c0 = (BM / 2) * ch + r16;
+    const int q_lo = FMT == FMT_MXFP4 ? g ^ swz_b<FMT>(r16) : (2 * g) ^ swz_b<FMT>(r16);
+    const int q_hi = FMT == FMT_MXFP4 ? (4 + g) ^ swz_b<FMT>(r16) : (2 * g + 1) ^ swz_b<FMT>(r16);
+    const uint8_t* const x_lo = st + L::kA + c0 * 128 + q_lo * 16;
+    const uint8_t* const x_hi = st + L::kA + c0 * 128 + q_hi * 16;
+    const uint8_t* const x_sc = sg + L::kWS + (FMT == FMT_FP8 ? c0 * 16 + sq * 4 : c0 * 4 + sq);
     auto read_x = [&](int i, i32x8& xf, uint32_t& xs) {
       const u32x4 lo = *reinterpret_cast<const u32x4*>(x_lo + 2048 * i);
       const u32x4 hi = *reinterpret_cast<const u32x4*>(x_hi + 2048 * i);
       xf = i32x8{(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
-      xs = *reinterpret_cast<const uint32_t*>(x_sc + 64 * i);
+      if constexpr (FMT == FMT_FP8) xs = *reinterpret_cast<const uint32_t*>(x_sc + 256 * i);
+      else if constexpr (FMT == FMT_MXFP4) xs = x_sc[64 * i];
     };
     // The next column tile's LDS reads are issued before this tile's MFMAs.
     // FP8: each scale fold is written kFoldLag MFMAs after its own MFMA (its
@@ -833,8 +875,8 @@ __global__ void __launch_bounds__(kQThreads) prefill_qgemm_kernel(PrefillGemmArg
     // waiting out the MFMA result latency; pin() keeps the accumulator updates
     // in that order.
     i32x8 xf[2];
-    uint32_t xs[2];
-    if constexpr (FMT == FMT_FP8) {
+    uint32_t xs[2] = {0u, 0u};
+    if constexpr (FMT != FMT_MXFP4) {
       // The step's first MFMA needs row tile 0 and column tile 0 only: those
       // reads are issued first (LDS returns in order), so after the barrier
       // each wave waits for four reads instead of the whole step's weight
@@ -860,13 +902,25 @@ __global__ void __launch_bounds__(kQThreads) prefill_qgemm_kernel(PrefillGemmArg
       fq[q] = 0.f;
     }
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < NCT; ++i) {
       if (ikb >= 0) {
 #pragma unroll
-        for (int q = 2 * i; q < 2 * i + 2; ++q)
+        for (int q = kPer * i; q < kPer * i + kPer; ++q)
           if (q < kPieces) issue_piece(q, ikb, istg);
       }
-      if (i + 1 < 8) read_x(i + 1, xf[(i + 1) & 1], xs[(i + 1) & 1]);
+      if (i + 1 < NCT) read_x(i + 1, xf[(i + 1) & 1], xs[(i + 1) & 1]);
+      if constexpr (FMT == FMT_BF16) {
+        // two K = 32 MFMAs per tile pair, the dependent one four MFMAs later
+        const auto half = [](const i32x8& r, int h) {
+          return __builtin_bit_cast(bf16x8, i32x4{r[4 * h], r[4 * h + 1], r[4 * h + 2], r[4 * h + 3]});
+        };
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(half(wf[j], h), half(xf[i & 1], h), acc[j][i], 0, 0, 0);
+        continue;
+      }
       // FP8 fold factors of this column tile: a weight scale covers 128 rows,
       // so tiles j = 0, 1 (gate rows) share one and tiles 2, 3 (up rows)
       // another, and the down GEMM's 64 rows of a wave share one
@@ -891,7 +945,7 @@ __global__ void __launch_bounds__(kQThreads) prefill_qgemm_kernel(PrefillGemmArg
           }
           tq[k % P] = t;
           fq[k % P] = fi[j >> 1];
-        } else {
+        } else if constexpr (FMT == FMT_MXFP4) {
           acc[j][i] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf[j], xf[i & 1], acc[j][i], 4, 0, 0, wcode[j], 0,
                                                                        static_cast<int>(xs[i & 1]));
         }
@@ -899,28 +953,28 @@ __global__ void __launch_bounds__(kQThreads) prefill_qgemm_kernel(PrefillGemmArg
     }
     if constexpr (FMT == FMT_FP8) {
 #pragma unroll
-      for (int k = 32 - P; k < 32; ++k) acc[k & 3][k >> 2] += tq[k % P] * fq[k % P];
+      for (int k = 4 * NCT - P; k < 4 * NCT; ++k) acc[k & 3][k >> 2] += tq[k % P] * fq[k % P];
     }
   };
 
-  // ---- epilogue: lane holds rows trow + g*4 + v of route column 128ch + 16i + r16
+  // ---- epilogue: lane holds rows trow + g*4 + v of route column (BM/2)ch + 16i + r16
   // (stg: an LDS stage that no copy targets before the next tile's K loop)
   auto epilogue = [&](const QTile& t, int b, uint8_t* stg) {
     const int n0 = n0_of(t);
+    const int lim_col = col_limit(t);
     if constexpr (GATE_UP) {
       // SwiGLU, then the down GEMM's activation quantisation of this 128-feature
       // group (one K group of the down GEMM) per route: amax over the 32 features
       // of the wave (lanes g = 0..3 of a column) and over the 4 row groups (LDS).
-      constexpr int QMODE = FMT == FMT_FP8 ? 0 : 2;
-      uint32_t pk[8][2][2];  // bf16 pairs (v0,v1), (v2,v3) of each column tile and gate/up tile pair
-      float amax[8];
+      uint32_t pk[NCT][2][2];  // bf16 pairs (v0,v1), (v2,v3) of each column tile and gate/up tile pair
+      float amax[NCT];
       // SiLU (every configuration here) runs as straight-line code with its
       // kind and the clamp of a clamped SwiGLU fixed at compile time; the other
       // kinds keep the runtime choice
       const float lim = t.shared ? a.sh_act_limit : a.act_limit;
       auto swiglu = [&](auto kind, auto clamp) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
+        for (int i = 0; i < NCT; ++i) {
           float m = 0.f;
 #pragma unroll
           for (int s2 = 0; s2 < 2; ++s2) {
@@ -943,12 +997,15 @@ __global__ void __launch_bounds__(kQThreads) prefill_qgemm_kernel(PrefillGemmArg
             for (int h = 0; h < 2; ++h) {
               const uint32_t p2 = pack_bf16x2(o[2 * h], o[2 * h + 1]);
               pk[i][s2][h] = p2;
-              m = fmaxf(m, fmaxf(fabsf(__uint_as_float(p2 << 16)), fabsf(__uint_as_float(p2 & 0xffff0000u))));
+              if constexpr (kQuant)
+                m = fmaxf(m, fmaxf(fabsf(__uint_as_float(p2 << 16)), fabsf(__uint_as_float(p2 & 0xffff0000u))));
             }
           }
-          m = fmaxf(m, __shfl_xor(m, 16));
-          m = fmaxf(m, __shfl_xor(m, 32));
-          amax[i] = m;
+          if constexpr (kQuant) {
+            m = fmaxf(m, __shfl_xor(m, 16));
+            m = fmaxf(m, __shfl_xor(m, 32));
+            amax[i] = m;
+          }
         }
       };
       if (a.act_kind == ACT_SILU) {
@@ -957,40 +1014,54 @@ __global__ void __launch_bounds__(kQThreads) prefill_qgemm_kernel(PrefillGemmArg
       } else {
         swiglu(std::integral_constant<int, -1>{}, std::false_type{});
       }
+      if constexpr (kQuant) {
+        constexpr int QMODE = FMT == FMT_FP8 ? 0 : 1;
+        float* const s_amax = reinterpret_cast<float*>(stg);  // [row group][column]
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
-        if (g == 0) s_amax[rg * kQBM + 128 * ch + 16 * i + r16] = amax[i];
-      // publish the amax (LDS only: the next tile's copies stay in flight)
-      wait_lgkm0();
-      bare_barrier();
-      const int ng = a.inter / 128;
+        for (int i = 0; i < NCT; ++i)
+          if (g == 0) s_amax[rg * BM + (BM / 2) * ch + 16 * i + r16] = amax[i];
+        // publish the amax (LDS only: the next tile's copies stay in flight)
+        wait_lgkm0();
+        bare_barrier();
+        const int sst = act_scale_stride(a.inter);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int col = 128 * ch + 16 * i + r16;
-        const int route = s_route[b][col];
-        if (route < 0) continue;
-        const float m =
-            fmaxf(fmaxf(s_amax[col], s_amax[kQBM + col]), fmaxf(s_amax[2 * kQBM + col], s_amax[3 * kQBM + col]));
-        float mul;
-        const float sc = group_scale<QMODE>(m, mul);
-        const int arow = t.shared ? a.numel + route : route;
+        for (int i = 0; i < NCT; ++i) {
+          const int col = (BM / 2) * ch + 16 * i + r16;
+          const int route = s_route[b][col];
+          if (route >= lim_col) continue;
+          const float m = fmaxf(fmaxf(s_amax[col], s_amax[BM + col]), fmaxf(s_amax[2 * BM + col], s_amax[3 * BM + col]));
+          float mul;
+          const float sc = group_scale<QMODE>(m, mul);
+          const int arow = t.shared ? a.numel + route : route;
 #pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2) {
-          float vals[4];
+          for (int s2 = 0; s2 < 2; ++s2) {
+            float vals[4];
 #pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            vals[2 * h] = quant_value<QMODE>(bf16_to_f32(static_cast<uint16_t>(pk[i][s2][h] & 0xffffu)), sc, mul);
-            vals[2 * h + 1] = quant_value<QMODE>(bf16_to_f32(static_cast<uint16_t>(pk[i][s2][h] >> 16)), sc, mul);
+            for (int h = 0; h < 2; ++h) {
+              vals[2 * h] = quant_value<QMODE>(bf16_to_f32(static_cast<uint16_t>(pk[i][s2][h] & 0xffffu)), sc, mul);
+              vals[2 * h + 1] = quant_value<QMODE>(bf16_to_f32(static_cast<uint16_t>(pk[i][s2][h] >> 16)), sc, mul);
+            }
+            uint32_t q4 = static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(vals[0], vals[1], 0, false));
+            q4 = static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(vals[2], vals[3], static_cast<int>(q4), true));
+            const int n = n0 + 32 * rg + 16 * s2 + g * 4;
+            *reinterpret_cast<uint32_t*>(a.act_q + static_cast<size_t>(arow) * a.inter + n) = q4;
           }
-          uint32_t q4 = static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(vals[0], vals[1], 0, false));
-          q4 = static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(vals[2], vals[3], static_cast<int>(q4), true));
-          const int n = n0 + 32 * rg + 16 * s2 + g * 4;
-          *reinterpret_cast<uint32_t*>(a.act_q + static_cast<size_t>(arow) * a.inter + n) = q4;
+          if (rg == 0 && g == 0) {
+            const size_t at = static_cast<size_t>(arow) * sst + t.ntile;
+            if (QMODE == 0) static_cast<float*>(a.act_s)[at] = sc;
+            else static_cast<uint8_t*>(a.act_s)[at] = static_cast<uint8_t>(sc);
+          }
         }
-        if (rg == 0 && g == 0) {
-          const size_t at = static_cast<size_t>(arow) * ng + t.ntile;
-          if (QMODE == 0) static_cast<float*>(a.act_s)[at] = sc;
-          else static_cast<uint32_t*>(a.act_s)[at] = static_cast<uint32_t>(sc);
+      } else {
+#pragma unroll
+        for (int i = 0; i < NCT; ++i) {
+          const int route = s_route[b][(BM / 2) * ch + 16 * i + r16];
+          if (route >= lim_col) continue;
+          const int arow = t.shared ? a.numel + route : route;
+#pragma unroll
+          for (int s2 = 0; s2 < 2; ++s2)
+            *reinterpret_cast<uint2*>(a.out + static_cast<size_t>(arow) * a.inter + n0 + 32 * rg + 16 * s2 + g * 4) =
+                uint2{pk[i][s2][0], pk[i][s2][1]};
         }
       }
     } else {
@@ -1002,19 +1073,19 @@ __global__ void __launch_bounds__(kQThreads) prefill_qgemm_kernel(PrefillGemmArg
       // of this wave's 64 output rows, 8 routes per instruction: half the
       // store instructions and a quarter of the memory requests.  N is a
       // multiple of 128, so a wave's rows are all inside N or all past it.
-      constexpr int CT = FMT == FMT_FP8 ? 4 : 2;
-      static_assert(8 * 16 * CT * 128 <= L::kStage, "a pass's staging areas fit one stage");
+      constexpr int CT = L::kStage >= 65536 ? 4 : L::kStage >= 32768 ? 2 : 1;
+      static_assert(8 * 16 * CT * 128 <= L::kStage && NCT % CT == 0, "a pass's staging areas fit one stage");
       uint8_t* const mine = stg + wave * (16 * CT * 128);
       const int nrow0 = n0 + 64 * rg;
       const bool rows_in = nrow0 < a.N;
       uint16_t* const base = t.shared ? a.sh_out : a.out;
 #pragma unroll
-      for (int p = 0; p < 8 / CT; ++p) {
+      for (int p = 0; p < NCT / CT; ++p) {
 #pragma unroll
         for (int ii = 0; ii < CT; ++ii) {
           const int i = p * CT + ii;
           const int c = 16 * ii + r16;  // staging row of this lane's route
-          const float wt = s_wt[b][128 * ch + 16 * i + r16];
+          const float wt = t.shared ? 1.0f : s_wt[b][(BM / 2) * ch + 16 * i + r16];
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
             uint2 pk2;
@@ -1031,9 +1102,13 @@ __global__ void __launch_bounds__(kQThreads) prefill_qgemm_kernel(PrefillGemmArg
         for (int kk = 0; kk < 2 * CT; ++kk) {
           const int c = 8 * kk + (lane >> 3), chunk = lane & 7;
           const u32x4 v = *reinterpret_cast<const u32x4*>(mine + c * 128 + ((chunk ^ (c & 7)) * 16));
-          const int route = s_route[b][128 * ch + 16 * (p * CT + (c >> 4)) + (c & 15)];
-          if (route >= 0 && rows_in)
-            *reinterpret_cast<u32x4*>(base + static_cast<size_t>(route) * a.N + nrow0 + 8 * chunk) = v;
+          const int route = s_route[b][(BM / 2) * ch + 16 * (p * CT + (c >> 4)) + (c & 15)];
+          if (route < lim_col && rows_in) {
+            u32x4* const dst = reinterpret_cast<u32x4*>(base + static_cast<size_t>(route) * a.N + nrow0 + 8 * chunk);
+            // (256-route tiles mean outputs far beyond L2: 8192 tokens, H 7168: down and combine 1% faster)
+            if constexpr (BM == 256) __builtin_nontemporal_store(v, dst);
+            else *dst = v;
+          }
         }
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
@@ -1041,75 +1116,97 @@ __global__ void __launch_bounds__(kQThreads) prefill_qgemm_kernel(PrefillGemmArg
     }
   };
 
+  // ---- route lists.  The column routes of a tile (its align entries) and, for
+  // the down GEMM, their router weights (setup) come by LDS-DMA too, so that no
+  // wait of an ordinary load drains the copies in flight.
+  auto fetch_routes = [&](const QTile& t, int b) {  // columns [64 wave, +64) by waves below BM/64
+    if (wave >= BM / 64) return;
+    const int ln = fresh_lane();
+    if (t.shared) {
+      s_route[b][64 * wave + ln] = t.mblock * BM + 64 * wave + ln;
+    } else {
+      const __amdgpu_buffer_rsrc_t rs = make_rsrc(a.sorted + static_cast<size_t>(t.mblock) * BM, BM * 4);
+      lds_buf4(rs, reinterpret_cast<uint8_t*>(&s_route[b][64 * wave]), (64 * wave + ln) * 4, 0);
+    }
+  };
+
   // ---- persistent loop over this workgroup's tiles (v, v + grid, ...).  The
   // K pipeline runs over a ring of S LDS stages with copies D steps ahead; the
   // ring continues across tiles (global step g0 + kb), so the last D steps of a
   // tile issue the next tile's first D steps, which land while this tile's
-  // epilogue runs.  The next tile's align entries are loaded at the start of
-  // a tile and published before its last D steps.
-  if (tid < kQBM) {
-    const int raw0 = raw_of(cur);
-    put_rows(cur, raw0, wt_of(cur, raw0), 0);
-  }
+  // epilogue runs.  The next tile's route list is copied at the start of a
+  // tile and has landed (and been published by a step's barrier) before its
+  // last D steps.
+  fetch_routes(cur, 0);
+  wait_vm<0>();
   __syncthreads();
   setup(cur, 0);
-  int buf = 0, g0 = 0;
+  int buf = 0, g0 = 0, gb = 0;  // gb: the tile's first scale group
   bool ahead = false;  // this tile's first D steps were issued during the previous tile
   for (;;) {
     if (!ahead) {
 #pragma unroll
       for (int d = 0; d < D; ++d)
-        if (d < nkb) issue(d, (g0 + d) % S);
+        if (d < nkb) issue(d, (g0 + d) % S, gb);
     }
     QTile nxt;
-    const bool has_next = map_tile_q<kChunk>(a, v + static_cast<int>(gridDim.x), nxt);
-    const bool cross = has_next && nkb > D;  // the next tile's first steps ride in this tile's last D steps
+    const bool has_next = map_tile_q<kChunk>(a, s_blk, v + static_cast<int>(gridDim.x), nxt);
+    // the next tile's first steps ride in this tile's last D steps, unless its
+    // first scale group's buffer would still be in use (kGroups 2 and a last
+    // group shorter than D)
+    const bool cross = has_next && nkb > D && (L::kGroups > 2 || (nkb & 3) == 0 || (nkb & 3) >= D);
+    const int gbn = gb + ngrp;
     // (pinned: a known-zero accumulator would let the compiler schedule the
     // first step, which it peels, apart from the others, at a register cost)
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
+      for (int i = 0; i < NCT; ++i) {
         acc[j][i] = zero;
         pin(acc[j][i]);
       }
-    wait_vm<0>();
+    // step 0 has landed once at most the copies of the D - 1 later steps (and
+    // nothing older) are outstanding; what the previous epilogue stored is
+    // newer than the copies and counts with them
+    if (nkb >= D) wait_vm<(D - 1) * L::kDmaPerStep>();
+    else wait_vm<0>();
     bare_barrier();
-    const int raw = has_next && tid < kQBM ? raw_of(nxt) : 0;
-    const float wraw = has_next && tid < kQBM ? wt_of(nxt, raw) : 1.0f;
+    if (has_next) fetch_routes(nxt, buf ^ 1);
     // steady steps: step kb + D of this tile is issued; step kb + 1 must have
     // landed at the end (later ones may still fly); every LDS read of the step
     // has returned before its MFMA used it
     int kb = 0;
     for (; kb < nkb - D; ++kb) {
       if constexpr (kSpread) {
-        compute((g0 + kb) % S, kb + D, (g0 + kb + D) % S);
+        compute(kb, (g0 + kb) % S, gb, kb + D, (g0 + kb + D) % S, gb);
       } else {
-        issue(kb + D, (g0 + kb + D) % S);
-        compute((g0 + kb) % S, -1, 0);
+        issue(kb + D, (g0 + kb + D) % S, gb);
+        compute(kb, (g0 + kb) % S, gb, -1, 0, 0);
       }
-      if (D == 2 && (kb + 2 < nkb || cross)) wait_vm<L::kDmaPerStep>();
-      else wait_vm<0>();
+      wait_vm<(D - 1) * L::kDmaPerStep>();
       wait_lgkm0();
       bare_barrier();
     }
-    // publish the next tile's rows; its first steps ride in this tile's last
-    // D steps
-    if (has_next) {
-      if (tid < kQBM) put_rows(nxt, raw, wraw, buf ^ 1);
+    // The next tile's routes were copied before step D's copies, so from
+    // nkb = 2D on the waits above covered them (at least D steady steps);
+    // shorter tiles wait for them here.  (Its router weights are copied by
+    // setup, before the copies of its first steps, and so have landed with the
+    // first of those.)
+    if (has_next && nkb < 2 * D) {
+      wait_vm<0>();
       wait_lgkm0();
       bare_barrier();
-      if (cross) setup(nxt, buf ^ 1);
     }
+    if (cross) setup(nxt, buf ^ 1);
     for (; kb < nkb; ++kb) {
       if constexpr (kSpread) {
-        compute((g0 + kb) % S, cross ? kb + D - nkb : -1, (g0 + kb + D) % S);
+        compute(kb, (g0 + kb) % S, gb, cross ? kb + D - nkb : -1, (g0 + kb + D) % S, gbn);
       } else {
-        if (cross) issue(kb + D - nkb, (g0 + kb + D) % S);
-        compute((g0 + kb) % S, -1, 0);
+        if (cross) issue(kb + D - nkb, (g0 + kb + D) % S, gbn);
+        compute(kb, (g0 + kb) % S, gb, -1, 0, 0);
       }
       if (kb + 1 < nkb) {
-        if (D == 2 && cross) wait_vm<L::kDmaPerStep>();
+        if (cross) wait_vm<(D - 1) * L::kDmaPerStep>();
         else wait_vm<0>();
       }
       wait_lgkm0();
@@ -1124,20 +1221,19 @@ __global__ void __launch_bounds__(kQThreads) prefill_qgemm_kernel(PrefillGemmArg
     cur = nxt;
     buf ^= 1;
     g0 += nkb;
+    gb = gbn % L::kGroups;
     v += static_cast<int>(gridDim.x);
     if (!ahead) setup(cur, buf);
   }
 }
 
-hipError_t launch_act_quant(int mode, const uint16_t* x, int rows, int K, uint8_t* q, void* scales,
+hipError_t launch_act_quant(int mode, const uint16_t* x, int rows, int K, int sstride, uint8_t* q, void* scales,
                             hipStream_t stream) {
   const dim3 grid((rows + 3) / 4), block(256);
   if (mode == 0)
-    hipLaunchKernelGGL(act_quant_kernel<0>, grid, block, 0, stream, x, rows, K, q, scales);
-  else if (mode == 1)
-    hipLaunchKernelGGL(act_quant_kernel<1>, grid, block, 0, stream, x, rows, K, q, scales);
+    hipLaunchKernelGGL(act_quant_kernel<0>, grid, block, 0, stream, x, rows, K, q, scales, sstride);
   else
-    hipLaunchKernelGGL(act_quant_kernel<2>, grid, block, 0, stream, x, rows, K, q, scales);
+    hipLaunchKernelGGL(act_quant_kernel<1>, grid, block, 0, stream, x, rows, K, q, scales, sstride);
   return hipGetLastError();
 }
 
@@ -1168,12 +1264,15 @@ static int q_cu_count() {
   return cached;
 }
 
-template <int FMT, int GU>
+template <int FMT, int GU, int BM>
 static hipError_t launch_qgemm_t(PrefillGemmArgs a, hipStream_t stream) {
+  // the ring, the scale groups, then one int per expert (and the total)
+  const int lds = QLds<FMT, BM>::kFixed + (a.num_experts + 1) * 4;
   static bool attr = false;
   if (!attr) {
-    const hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_qgemm_kernel<FMT, GU>),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, QLds<FMT>::kTotal);
+    const hipError_t err =
+        hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_qgemm_kernel<FMT, GU, BM>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 4096);
     if (err != hipSuccess) return err;
     attr = true;
   }
@@ -1184,14 +1283,22 @@ static hipError_t launch_qgemm_t(PrefillGemmArgs a, hipStream_t stream) {
   const long long tiles = static_cast<long long>(a.max_blocks + a.shared_blocks) * a.ntiles;
   const int wgs = static_cast<int>(std::min<long long>(tiles, q_cu_count()));
   if (wgs <= 0) return hipSuccess;
-  hipLaunchKernelGGL((prefill_qgemm_kernel<FMT, GU>), dim3(wgs), dim3(kQThreads), QLds<FMT>::kTotal, stream, a);
+  hipLaunchKernelGGL((prefill_qgemm_kernel<FMT, GU, BM>), dim3(wgs), dim3(kQThreads), lds, stream, a);
   return hipGetLastError();
 }
 
+template <int FMT, int GU>
+static hipError_t launch_qgemm_bm(const PrefillGemmArgs& a, hipStream_t stream) {
+  if (a.block == 64) return launch_qgemm_t<FMT, GU, 64>(a, stream);
+  if (a.block == 128) return launch_qgemm_t<FMT, GU, 128>(a, stream);
+  if (a.block == 256) return launch_qgemm_t<FMT, GU, 256>(a, stream);
+  return hipErrorInvalidValue;
+}
+
 hipError_t launch_prefill_gemm(int fmt, int gate_up, const PrefillGemmArgs& a, hipStream_t stream) {
-  if (fmt == FMT_FP8) return gate_up ? launch_qgemm_t<FMT_FP8, 1>(a, stream) : launch_qgemm_t<FMT_FP8, 0>(a, stream);
+  if (fmt == FMT_FP8) return gate_up ? launch_qgemm_bm<FMT_FP8, 1>(a, stream) : launch_qgemm_bm<FMT_FP8, 0>(a, stream);
   if (fmt == FMT_MXFP4)
-    return gate_up ? launch_qgemm_t<FMT_MXFP4, 1>(a, stream) : launch_qgemm_t<FMT_MXFP4, 0>(a, stream);
+    return gate_up ? launch_qgemm_bm<FMT_MXFP4, 1>(a, stream) : launch_qgemm_bm<FMT_MXFP4, 0>(a, stream);
   if (fmt == FMT_BF16) return gate_up ? launch_gemm_t<FMT_BF16, 1>(a, stream) : launch_gemm_t<FMT_BF16, 0>(a, stream);
   return hipErrorInvalidValue;
 }

@@ -6,8 +6,7 @@
 //   MODE 0: float scale s = max(amax, 1e-10) / 448, q = e4m3(clamp(x / s))
 //           (reference per_token_group_quant_fp8, kernel/triton/fp8_block_linear.py:53-59)
 //   MODE 1: e8m0 scale 2^ceil(log2(max(amax, 1e-4) * (1/448))), q = e4m3(x / 2^e),
-//           codes stored as uint8; MODE 2: the same with codes stored as uint32
-//           (the grouped GEMM copies them to LDS in 4-byte units)
+//           codes stored as uint8
 #pragma once
 
 #include "ftmoe_common.h"
@@ -17,7 +16,7 @@ namespace ftmoe {
 // Scale of one group with absolute maximum amax.
 // MODE 0: returns s and sets mul = RN(1/s), the rounded reciprocal that
 // quant_value's division uses;
-// MODE 1/2: returns the e8m0 code e+127 as a float and sets mul = 2^-e.
+// MODE 1: returns the e8m0 code e+127 as a float and sets mul = 2^-e.
 template <int MODE>
 __device__ __forceinline__ float group_scale(float amax, float& mul) {
   if (MODE == 0) {

@@ -125,3 +125,33 @@ def test_prefill_activation_variants(dev, fmt, activation):
     assert cosine(got, y_ref) >= COS_TOL, (fmt, activation, cosine(got, y_ref))
     y_silu = oracle.experts.moe_layer("prefill", x, w, ids, bank, sh)
     assert max_rel(y_silu, y_ref) > 4 * MAX_REL_TOL
+
+
+@pytest.mark.parametrize("H,I", [(640, 384), (128, 1152), (1024, 128)])
+@pytest.mark.parametrize("block,E,E2", [(64, 16, 3), (128, 4, 16), (256, 4, 16)])
+@pytest.mark.parametrize("fmt", ["fp8", "mxfp4"])
+def test_prefill_block_sizes(dev, fmt, block, E, E2, H, I):
+    """Every routes-per-tile variant of the quantised GEMMs at its edges: one
+    expert with a full block, one with a route more, one with a single route,
+    the rest empty (the mean over the E bank rows picks the variant); K of 1,
+    3, 5, 8 and 9 steps: shorter than the copies run ahead, whole and partial
+    groups of scales.  The tiling does not enter an output's arithmetic, so the
+    same call over E2 rows, which takes another variant, gives the same bits.
+    The oracle is held by its 2-norm: with these short K a single activation
+    whose bf16 rounding, and with it its e4m3 code, falls the other way (the
+    sums differ in their last bit) moves one output row by up to 1/16 of that
+    product, which the maximum over few outputs would show as 2-3%."""
+    rng = np.random.default_rng(block + H)
+    flat = np.repeat(np.arange(3, dtype=np.int32), [block, block + 1, 1])
+    ids = rng.permutation(flat).reshape(-1, 2)
+    M = ids.shape[0]
+    w = rng.uniform(0.1, 1.0, size=ids.shape).astype(np.float32)
+    bank, sh = synth.make_bank(fmt, 16, H, I, rng), synth.make_bank(fmt, 1, H, I, rng)
+    x = synth.activations(rng, M, H)
+    y_ref = oracle.experts.moe_layer("prefill", x, w, ids, bank, sh)
+    y, y2 = (ops.experts_prefill(bf16_dev(x, dev), torch.from_numpy(w).to(dev), torch.from_numpy(ids).to(dev),
+                                 to_device_bank(bank, dev, slice(0, n)), to_device_bank(sh, dev)) for n in (E, E2))
+    assert torch.equal(y, y2)
+    got = to_np(y).astype(np.float64)
+    assert np.linalg.norm(got - y_ref) <= 1e-2 * np.linalg.norm(y_ref)
+    assert cosine(got, y_ref) >= COS_TOL, cosine(got, y_ref)
