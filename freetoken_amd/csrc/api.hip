@@ -697,10 +697,11 @@ int ftmoe_experts_prefill(const void* x, int M, int top_k, const float* topk_w, 
   const int numel = M * top_k;
   const int H = bank->hidden, I = bank->inter;
   const int fmt = bank->format;
-  // the quantised GEMMs address each operand (activations, one expert's
-  // weights) through a buffer descriptor with 31-bit offsets
-  if (fmt != FTMOE_FMT_BF16 && (static_cast<int64_t>(numel + M) * I > INT32_MAX ||
-                                static_cast<int64_t>(M) * H > INT32_MAX || 2 * static_cast<int64_t>(I) * H > INT32_MAX))
+  // the LDS-DMA GEMMs address each operand (activations, one expert's
+  // weights) through a buffer descriptor with 31-bit offsets; bf16 calls beyond
+  // that take the register-staged GEMM
+  const bool fits = ftmoe::prefill_operands_fit(fmt, M, top_k, H, I);
+  if (fmt != FTMOE_FMT_BF16 && !fits)
     return fail(FTMOE_ERR_UNSUPPORTED, "experts_prefill: an operand beyond 2 GiB (M=%d top_k=%d H=%d I=%d)", M,
                 top_k, H, I);
 
@@ -738,6 +739,7 @@ int ftmoe_experts_prefill(const void* x, int M, int top_k, const float* topk_w, 
   g.k = top_k;
   g.k_magic = top_k == 1 ? 0u : static_cast<uint32_t>(((uint64_t{1} << 32) + top_k - 1) / top_k);
   g.block = bm;
+  g.wide = !fits;
   g.max_blocks = L.max_blocks;
   g.shared_blocks = shared ? (M + bm - 1) / bm : 0;
   g.w = {nullptr, nullptr};

@@ -133,6 +133,7 @@ struct PrefillGemmArgs {
   int M, k;
   uint32_t k_magic;         // ceil(2^32 / k), 0 for k = 1: r / k = umulhi(r, k_magic) for r < 2^26
   int block;                // routes per M block (BM)
+  int wide;                 // bf16: an operand beyond 2 GiB (prefill_operands_fit is false)
   int max_blocks;           // routed M blocks of the grid
   int shared_blocks;        // ceil(M / BM) if a shared expert is present, else 0
   int ntiles;               // N tiles
@@ -154,9 +155,17 @@ struct PrefillGemmArgs {
 
 constexpr int kPrefillMaxRows = 1023;  // bank rows of a prefill call
 
-// Routes per M block of the prefill GEMMs (the align block size).  bf16: 128.
-// Quantised formats: 256, or by the mean number of routes per expert r = M k /
-// rows 64 (r <= 48) or 128 (r <= 120): a tile of 256 is then mostly padding.
+// Whether every operand of a prefill call (activations, one expert's weights)
+// fits the 31-bit offsets of the LDS-DMA GEMM's buffer descriptors.
+inline bool prefill_operands_fit(int fmt, int M, int k, int H, int I) {
+  const long long b = fmt == FMT_BF16 ? 2 : 1, lim = INT32_MAX;
+  return (static_cast<long long>(M) * k + M) * I * b <= lim && static_cast<long long>(M) * H * b <= lim &&
+         2ll * I * H * b <= lim;
+}
+
+// Routes per M block of the prefill GEMMs (the align block size): 256, or by
+// the mean number of routes per expert r = M k / rows 64 (r <= 48) or 128 (r <=
+// 120; bf16 r <= 320): a tile of 256 is then mostly padding.
 // Measured (us, blocks of 64 / 128 / 256): FP8 H 2048, I 768, 128 experts,
 // top-8, r = 31 165 / 172 / 206, r = 69 214 / 189 / 223, r = 112 252 / 223 /
 // 239, r = 137 287 / 263 / 243; MXFP4 of that shape r = 31 118 / 130 / 179, r =
@@ -164,14 +173,17 @@ constexpr int kPrefillMaxRows = 1023;  // bank rows of a prefill call
 // experts, r = 35 502 / 504 / 736, r = 75 713 / 638 / 790.  Uneven routings move
 // the upper line outwards (FP8 H 7168, I 2048, 256 experts, r = 125 3512 / 2971
 // / 3303), but at r = 137 an even one is already 8% slower at 128.
+// bf16 of the first shape: r = 38 267 / 271 / 311, r = 87 355 / 302 / 338, r =
+// 256 628 / 487 / 507 (uneven 647 / 515 / 564), r = 512 1115 / 825 / 803.
 // The MXFP4 tiles of 256 hold two groups of scales, which costs their copies'
 // overlap across tiles when K / 128 leaves a remainder of 1 by four, and up to
 // 511 experts in LDS: 128 takes those calls.
 inline int prefill_block_size(int fmt, int M, int k, int rows, int H, int I) {
-  if (fmt == FMT_BF16) return 128;
+  // (the register-staged bf16 GEMM tiles 128)
+  if (fmt == FMT_BF16 && !prefill_operands_fit(fmt, M, k, H, I)) return 128;
   const long long routes = static_cast<long long>(M) * k;
   if (routes <= 48ll * rows) return 64;
-  if (routes <= 120ll * rows) return 128;
+  if (routes <= (fmt == FMT_BF16 ? 320ll : 120ll) * rows) return 128;
   if (fmt == FMT_MXFP4 && (rows > 511 || H / 128 % 4 == 1 || I / 128 % 4 == 1)) return 128;
   return 256;
 }

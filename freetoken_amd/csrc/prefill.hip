@@ -15,11 +15,13 @@
 //             scales in hardware and accumulates directly.
 //   FMT_BF16  bf16 activations and weights, v_mfma_f32_16x16x32_bf16.
 //
-// The quantised formats (FP8, MXFP4) run prefill_qgemm_kernel, whose tiling,
-// copies and schedule are described at its section below; the rest of this
-// header describes the bf16 grouped GEMM (prefill_gemm_kernel).
+// All three run prefill_qgemm_kernel, whose tiling, copies and schedule are
+// described at its section below.  bf16 calls with an operand beyond 2 GiB,
+// past the 31-bit offsets of that kernel's buffer descriptors, take the
+// register-staged prefill_gemm_kernel, which addresses with 64 bits; the rest
+// of this header describes it.
 //
-// Tiling (bf16): a workgroup computes a 128 (weight rows) x 128 (routes) tile with 4 waves
+// Tiling: a workgroup computes a 128 (weight rows) x 128 (routes) tile with 4 waves
 // (2 x 2), each 64 x 64 = 4 x 4 MFMA blocks.  Weights are the MFMA A operand, so a
 // lane's four accumulators are four consecutive output features of one route and
 // stores are 8-byte vectors.  K advances 128 per step; global->LDS copies of the
@@ -120,35 +122,11 @@ __global__ void __launch_bounds__(256) act_quant_kernel(const uint16_t* __restri
 // Grouped GEMM
 // ----------------------------------------------------------------------------
 
-template <int FMT>
-struct TileCfg;
-template <>
-struct TileCfg<FMT_FP8> {
-  static constexpr int kWRow = 128;  // bytes of a weight row per K step
-  static constexpr int kXRow = 128;
-};
-template <>
-struct TileCfg<FMT_MXFP4> {
-  static constexpr int kWRow = 64;
-  static constexpr int kXRow = 128;
-};
-template <>
-struct TileCfg<FMT_BF16> {
-  static constexpr int kWRow = 256;
-  static constexpr int kXRow = 256;
-};
-
-template <int FMT>
-struct Lds {
-  static constexpr int kWStride = TileCfg<FMT>::kWRow + 16;
-  static constexpr int kXStride = TileCfg<FMT>::kXRow + 16;
-  static constexpr int kW = kPBN * kWStride;
-  static constexpr int kX = kPBM * kXStride;
-  static constexpr int kWS = FMT == FMT_MXFP4 ? kPBN * 4 : 0;  // e8m0 codes, 4 per row per step
-  static constexpr int kXS = kPBM * 4;                          // float or e8m0 (one per row)
-  static constexpr int kBuf = kW + kX + kWS + kXS;
-  static constexpr int kTotal = 2 * kBuf;
-};
+constexpr int kPRow = 256;            // bytes of a weight or activation row per K step (128 values)
+constexpr int kPStride = kPRow + 16;  // LDS row stride
+constexpr int kPW = kPBN * kPStride;
+constexpr int kPBuf = kPW + kPBM * kPStride;
+constexpr int kPLds = 2 * kPBuf;
 
 // Maps a workgroup to (expert or shared, M block, N tile); returns false when idle.
 __device__ __forceinline__ bool map_tile(const PrefillGemmArgs& a, int wg, bool& shared, int& expert, int& mblock,
@@ -184,10 +162,8 @@ __device__ __forceinline__ bool map_tile(const PrefillGemmArgs& a, int wg, bool&
   return false;
 }
 
-template <int FMT, int GATE_UP>
+template <int GATE_UP>
 __global__ void __launch_bounds__(kPThreads) prefill_gemm_kernel(PrefillGemmArgs a) {
-  using L = Lds<FMT>;
-  using C = TileCfg<FMT>;
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
   __shared__ int s_row[kPBM];   // activation row of each tile column (-1: padding)
   __shared__ int s_route[kPBM]; // route (routed) or token (shared) of each column, -1: padding
@@ -224,10 +200,8 @@ __global__ void __launch_bounds__(kPThreads) prefill_gemm_kernel(PrefillGemmArgs
 
   const BankView bank = shared ? a.ws : a.w;
   const int n0 = GATE_UP ? ntile * (kPBN / 2) : ntile * kPBN;
-  const size_t wrow_bytes = FMT == FMT_BF16 ? static_cast<size_t>(a.K) * 2
-                            : FMT == FMT_FP8 ? static_cast<size_t>(a.K) : static_cast<size_t>(a.K) / 2;
-  const uint8_t* wexp = bank.w + static_cast<size_t>(expert) * a.N * wrow_bytes;
-  const size_t xrow_bytes = FMT == FMT_BF16 ? static_cast<size_t>(a.K) * 2 : static_cast<size_t>(a.K);
+  const size_t row_bytes = static_cast<size_t>(a.K) * 2;
+  const uint8_t* wexp = bank.w + static_cast<size_t>(expert) * a.N * row_bytes;
   const int nkb = a.K / 128;
 
   auto wrow_of = [&](int r) -> int {  // weight row held in tile row r
@@ -236,68 +210,43 @@ __global__ void __launch_bounds__(kPThreads) prefill_gemm_kernel(PrefillGemmArgs
   };
 
   // ---- global -> register staging of one K step
-  constexpr int kWChunks = kPBN * C::kWRow / 16;
-  constexpr int kXChunks = kPBM * C::kXRow / 16;
+  constexpr int kWChunks = kPBN * kPRow / 16;
+  constexpr int kXChunks = kPBM * kPRow / 16;
   constexpr int kWPer = kWChunks / kPThreads;
   constexpr int kXPer = kXChunks / kPThreads;
   u32x4 wreg[kWPer], xreg[kXPer];
-  uint32_t wsreg = 0;   // MXFP4: 4 e8m0 codes of one weight row (threads < BN)
-  uint32_t xsreg = 0;   // scale of one activation row (threads < BM), float bits or code
 
   auto load_step = [&](int kb) {
 #pragma unroll
     for (int q = 0; q < kWPer; ++q) {
       const int c = tid + q * kPThreads;
-      const int r = c / (C::kWRow / 16), col = c % (C::kWRow / 16);
-      const uint8_t* p = wexp + static_cast<size_t>(wrow_of(r)) * wrow_bytes + static_cast<size_t>(kb) * C::kWRow + col * 16;
+      const int r = c / (kPRow / 16), col = c % (kPRow / 16);
+      const uint8_t* p = wexp + static_cast<size_t>(wrow_of(r)) * row_bytes + static_cast<size_t>(kb) * kPRow + col * 16;
       wreg[q] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
     }
 #pragma unroll
     for (int q = 0; q < kXPer; ++q) {
       const int c = tid + q * kPThreads;
-      const int r = c / (C::kXRow / 16), col = c % (C::kXRow / 16);
+      const int r = c / (kPRow / 16), col = c % (kPRow / 16);
       const int row = s_row[r];
       const int src = row < 0 ? 0 : row;
-      const uint8_t* p = a.xq + static_cast<size_t>(src) * xrow_bytes + static_cast<size_t>(kb) * C::kXRow + col * 16;
+      const uint8_t* p = a.xq + static_cast<size_t>(src) * row_bytes + static_cast<size_t>(kb) * kPRow + col * 16;
       xreg[q] = *reinterpret_cast<const u32x4*>(p);
-    }
-    if constexpr (FMT == FMT_MXFP4) {
-      if (tid < kPBN) {
-        const uint8_t* sp = static_cast<const uint8_t*>(bank.s) +
-                            (static_cast<size_t>(expert) * a.N + wrow_of(tid)) * (a.K / 32) + kb * 4;
-        wsreg = *reinterpret_cast<const uint32_t*>(sp);
-      }
-    }
-    if constexpr (FMT != FMT_BF16) {
-      if (tid < kPBM) {
-        const int row = s_row[tid];
-        const int src = row < 0 ? 0 : row;
-        if (FMT == FMT_FP8)
-          xsreg = __float_as_uint(static_cast<const float*>(a.xs)[static_cast<size_t>(src) * nkb + kb]);
-        else
-          xsreg = static_cast<const uint8_t*>(a.xs)[static_cast<size_t>(src) * nkb + kb];
-      }
     }
   };
   auto store_step = [&](int buf) {
-    uint8_t* base = lds + buf * L::kBuf;
+    uint8_t* base = lds + buf * kPBuf;
 #pragma unroll
     for (int q = 0; q < kWPer; ++q) {
       const int c = tid + q * kPThreads;
-      const int r = c / (C::kWRow / 16), col = c % (C::kWRow / 16);
-      *reinterpret_cast<u32x4*>(base + r * L::kWStride + col * 16) = wreg[q];
+      const int r = c / (kPRow / 16), col = c % (kPRow / 16);
+      *reinterpret_cast<u32x4*>(base + r * kPStride + col * 16) = wreg[q];
     }
 #pragma unroll
     for (int q = 0; q < kXPer; ++q) {
       const int c = tid + q * kPThreads;
-      const int r = c / (C::kXRow / 16), col = c % (C::kXRow / 16);
-      *reinterpret_cast<u32x4*>(base + L::kW + r * L::kXStride + col * 16) = xreg[q];
-    }
-    if constexpr (FMT == FMT_MXFP4) {
-      if (tid < kPBN) *reinterpret_cast<uint32_t*>(base + L::kW + L::kX + tid * 4) = wsreg;
-    }
-    if constexpr (FMT != FMT_BF16) {
-      if (tid < kPBM) *reinterpret_cast<uint32_t*>(base + L::kW + L::kX + L::kWS + tid * 4) = xsreg;
+      const int r = c / (kPRow / 16), col = c % (kPRow / 16);
+      *reinterpret_cast<u32x4*>(base + kPW + r * kPStride + col * 16) = xreg[q];
     }
   };
 
@@ -324,82 +273,24 @@ __global__ void __launch_bounds__(kPThreads) prefill_gemm_kernel(PrefillGemmArgs
   for (int kb = 0; kb < nkb; ++kb) {
     const int cur = kb & 1;
     if (kb + 1 < nkb) load_step(kb + 1);
-    const uint8_t* base = lds + cur * L::kBuf;
+    const uint8_t* base = lds + cur * kPBuf;
 
-    if constexpr (FMT == FMT_FP8) {
-      float sw[4];
+    // four K=32 MFMAs per 128 step
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int wr = wrow_of(wrow_base[j]);
-        sw[j] = static_cast<const float*>(bank.s)[(static_cast<size_t>(expert) * (a.N / 128) + wr / 128) * nkb + kb];
-      }
-      i32x8 xf[4];
-      float sx[4];
+    for (int s = 0; s < 4; ++s) {
+      bf16x8 xf[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const uint8_t* p = base + L::kW + (xcol_base + 16 * i + r16) * L::kXStride + g * 32;
-        const u32x4 lo = *reinterpret_cast<const u32x4*>(p);
-        const u32x4 hi = *reinterpret_cast<const u32x4*>(p + 16);
-        xf[i] = i32x8{(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
-        sx[i] = *reinterpret_cast<const float*>(base + L::kW + L::kX + L::kWS + (xcol_base + 16 * i + r16) * 4);
+        const uint8_t* p = base + kPW + (xcol_base + 16 * i + r16) * kPStride + (g * 32 + s * 8) * 2;
+        xf[i] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(p));
       }
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const uint8_t* p = base + (wrow_base[j] + r16) * L::kWStride + g * 32;
-        const u32x4 lo = *reinterpret_cast<const u32x4*>(p);
-        const u32x4 hi = *reinterpret_cast<const u32x4*>(p + 16);
-        const i32x8 wf = {(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const f32x4 t = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf, xf[i], zero, 0, 0, 0, 0, 0, 0);
-          const float f = sx[i] * sw[j];
-          acc[j][i] += t * f;
-        }
-      }
-    } else if constexpr (FMT == FMT_MXFP4) {
-      // The f8f6f4 MFMA reads an fp8 lane-group g as K = 16g+[0,16) (bytes 0-15)
-      // and 64+16g+[0,16) (bytes 16-31), an fp4 lane-group g as the 32-value
-      // block [32g, 32g+32), and scale lane-group q as K block q.  The fp4
-      // weights are stored K-contiguous, so the fp8 activations are fed in that
-      // split order to pair every product with its K.
-      i32x8 xf[4];
-      int sxc[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const uint8_t* p = base + L::kW + (xcol_base + 16 * i + r16) * L::kXStride;
-        const u32x4 lo = *reinterpret_cast<const u32x4*>(p + 16 * g);
-        const u32x4 hi = *reinterpret_cast<const u32x4*>(p + 64 + 16 * g);
-        xf[i] = i32x8{(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
-        sxc[i] = static_cast<int>(*reinterpret_cast<const uint32_t*>(base + L::kW + L::kX + L::kWS +
-                                                                     (xcol_base + 16 * i + r16) * 4));
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const uint8_t* p = base + (wrow_base[j] + r16) * L::kWStride + g * 16;
-        const u32x4 v = *reinterpret_cast<const u32x4*>(p);
-        const i32x8 wf = {(int)v[0], (int)v[1], (int)v[2], (int)v[3], 0, 0, 0, 0};
-        const int swc = base[L::kW + L::kX + (wrow_base[j] + r16) * 4 + g];
+        const uint8_t* p = base + (wrow_base[j] + r16) * kPStride + (g * 32 + s * 8) * 2;
+        const bf16x8 wf = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(p));
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          acc[j][i] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(wf, xf[i], acc[j][i], 4, 0, 0, swc, 0, sxc[i]);
-      }
-    } else {  // FMT_BF16: four K=32 MFMAs per 128 step
-#pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        bf16x8 xf[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const uint8_t* p = base + L::kW + (xcol_base + 16 * i + r16) * L::kXStride + (g * 32 + s * 8) * 2;
-          xf[i] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(p));
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const uint8_t* p = base + (wrow_base[j] + r16) * L::kWStride + (g * 32 + s * 8) * 2;
-          const bf16x8 wf = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(p));
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, xf[i], acc[j][i], 0, 0, 0);
-        }
+          acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, xf[i], acc[j][i], 0, 0, 0);
       }
     }
 
@@ -919,6 +810,8 @@ __global__ void __launch_bounds__(kQThreads) prefill_qgemm_kernel(PrefillGemmArg
 #pragma unroll
           for (int j = 0; j < 4; ++j)
             acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(half(wf[j], h), half(xf[i & 1], h), acc[j][i], 0, 0, 0);
+        // (keeps the later tiles' reads from being hoisted into spills)
+        if constexpr (BM == 256) __builtin_amdgcn_sched_barrier(0);
         continue;
       }
       // FP8 fold factors of this column tile: a weight scale covers 128 rows,
@@ -966,7 +859,8 @@ __global__ void __launch_bounds__(kQThreads) prefill_qgemm_kernel(PrefillGemmArg
       // SwiGLU, then the down GEMM's activation quantisation of this 128-feature
       // group (one K group of the down GEMM) per route: amax over the 32 features
       // of the wave (lanes g = 0..3 of a column) and over the 4 row groups (LDS).
-      uint32_t pk[NCT][2][2];  // bf16 pairs (v0,v1), (v2,v3) of each column tile and gate/up tile pair
+      // bf16 pairs (v0,v1), (v2,v3) of each column tile and gate/up tile pair (bf16: stored at once)
+      uint32_t pk[kQuant ? NCT : 1][2][2];
       float amax[NCT];
       // SiLU (every configuration here) runs as straight-line code with its
       // kind and the clamp of a clamped SwiGLU fixed at compile time; the other
@@ -996,9 +890,17 @@ __global__ void __launch_bounds__(kQThreads) prefill_qgemm_kernel(PrefillGemmArg
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
               const uint32_t p2 = pack_bf16x2(o[2 * h], o[2 * h + 1]);
-              pk[i][s2][h] = p2;
+              pk[kQuant ? i : 0][s2][h] = p2;
               if constexpr (kQuant)
                 m = fmaxf(m, fmaxf(fabsf(__uint_as_float(p2 << 16)), fabsf(__uint_as_float(p2 & 0xffff0000u))));
+            }
+          }
+          if constexpr (!kQuant) {
+            const int route = s_route[b][(BM / 2) * ch + 16 * i + r16];
+            if (route < lim_col) {
+              uint16_t* const dst = a.out + static_cast<size_t>(t.shared ? a.numel + route : route) * a.inter + n0 + 32 * rg + g * 4;
+              *reinterpret_cast<uint2*>(dst) = uint2{pk[0][0][0], pk[0][0][1]};
+              *reinterpret_cast<uint2*>(dst + 16) = uint2{pk[0][1][0], pk[0][1][1]};
             }
           }
           if constexpr (kQuant) {
@@ -1051,17 +953,6 @@ __global__ void __launch_bounds__(kQThreads) prefill_qgemm_kernel(PrefillGemmArg
             if (QMODE == 0) static_cast<float*>(a.act_s)[at] = sc;
             else static_cast<uint8_t*>(a.act_s)[at] = static_cast<uint8_t>(sc);
           }
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < NCT; ++i) {
-          const int route = s_route[b][(BM / 2) * ch + 16 * i + r16];
-          if (route >= lim_col) continue;
-          const int arow = t.shared ? a.numel + route : route;
-#pragma unroll
-          for (int s2 = 0; s2 < 2; ++s2)
-            *reinterpret_cast<uint2*>(a.out + static_cast<size_t>(arow) * a.inter + n0 + 32 * rg + 16 * s2 + g * 4) =
-                uint2{pk[i][s2][0], pk[i][s2][1]};
         }
       }
     } else {
@@ -1237,17 +1128,17 @@ hipError_t launch_act_quant(int mode, const uint16_t* x, int rows, int K, int ss
   return hipGetLastError();
 }
 
-template <int FMT, int GU>
+template <int GU>
 static hipError_t launch_gemm_t(const PrefillGemmArgs& a, hipStream_t stream) {
   static bool attr = false;
-  const void* fn = reinterpret_cast<const void*>(prefill_gemm_kernel<FMT, GU>);
+  const void* fn = reinterpret_cast<const void*>(prefill_gemm_kernel<GU>);
   if (!attr) {
-    hipError_t err = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, Lds<FMT>::kTotal);
+    hipError_t err = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, kPLds);
     if (err != hipSuccess) return err;
     attr = true;
   }
   const int wgs = (a.max_blocks + a.shared_blocks) * a.ntiles;
-  hipLaunchKernelGGL((prefill_gemm_kernel<FMT, GU>), dim3(wgs), dim3(kPThreads), Lds<FMT>::kTotal, stream, a);
+  hipLaunchKernelGGL((prefill_gemm_kernel<GU>), dim3(wgs), dim3(kPThreads), kPLds, stream, a);
   return hipGetLastError();
 }
 
@@ -1299,7 +1190,9 @@ hipError_t launch_prefill_gemm(int fmt, int gate_up, const PrefillGemmArgs& a, h
   if (fmt == FMT_FP8) return gate_up ? launch_qgemm_bm<FMT_FP8, 1>(a, stream) : launch_qgemm_bm<FMT_FP8, 0>(a, stream);
   if (fmt == FMT_MXFP4)
     return gate_up ? launch_qgemm_bm<FMT_MXFP4, 1>(a, stream) : launch_qgemm_bm<FMT_MXFP4, 0>(a, stream);
-  if (fmt == FMT_BF16) return gate_up ? launch_gemm_t<FMT_BF16, 1>(a, stream) : launch_gemm_t<FMT_BF16, 0>(a, stream);
+  if (fmt == FMT_BF16 && a.wide) return gate_up ? launch_gemm_t<1>(a, stream) : launch_gemm_t<0>(a, stream);
+  if (fmt == FMT_BF16)
+    return gate_up ? launch_qgemm_bm<FMT_BF16, 1>(a, stream) : launch_qgemm_bm<FMT_BF16, 0>(a, stream);
   return hipErrorInvalidValue;
 }
 

@@ -128,21 +128,24 @@ def test_prefill_activation_variants(dev, fmt, activation):
 
 
 @pytest.mark.parametrize("H,I", [(640, 384), (128, 1152), (1024, 128)])
-@pytest.mark.parametrize("block,E,E2", [(64, 16, 3), (128, 4, 16), (256, 4, 16)])
-@pytest.mark.parametrize("fmt", ["fp8", "mxfp4"])
-def test_prefill_block_sizes(dev, fmt, block, E, E2, H, I):
-    """Every routes-per-tile variant of the quantised GEMMs at its edges: one
-    expert with a full block, one with a route more, one with a single route,
-    the rest empty (the mean over the E bank rows picks the variant); K of 1,
-    3, 5, 8 and 9 steps: shorter than the copies run ahead, whole and partial
-    groups of scales.  The tiling does not enter an output's arithmetic, so the
-    same call over E2 rows, which takes another variant, gives the same bits.
+@pytest.mark.parametrize("fmt,block,n,E,E2", [
+    ("fp8", 64, 1, 16, 3), ("fp8", 128, 1, 4, 16), ("fp8", 256, 1, 4, 16),
+    ("mxfp4", 64, 1, 16, 3), ("mxfp4", 128, 1, 4, 16), ("mxfp4", 256, 1, 4, 16),
+    ("bf16", 64, 1, 16, 3), ("bf16", 128, 1, 4, 16), ("bf16", 256, 2, 3, 16),
+])
+def test_prefill_block_sizes(dev, fmt, block, n, E, E2, H, I):
+    """Every routes-per-tile variant of the GEMMs at its edges: one expert with
+    n full blocks, one with a route more, one with a single route, the rest
+    empty (the mean over the E bank rows picks the variant); K of 1, 3, 5, 8 and
+    9 blocks of 128: shorter than the copies run ahead, whole and partial groups
+    of scales.  The tiling does not enter an output's arithmetic, so the same
+    call over E2 rows, which takes another variant, gives the same bits.
     The oracle is held by its 2-norm: with these short K a single activation
     whose bf16 rounding, and with it its e4m3 code, falls the other way (the
     sums differ in their last bit) moves one output row by up to 1/16 of that
     product, which the maximum over few outputs would show as 2-3%."""
     rng = np.random.default_rng(block + H)
-    flat = np.repeat(np.arange(3, dtype=np.int32), [block, block + 1, 1])
+    flat = np.repeat(np.arange(3, dtype=np.int32), [n * block, n * block + 1, 1])
     ids = rng.permutation(flat).reshape(-1, 2)
     M = ids.shape[0]
     w = rng.uniform(0.1, 1.0, size=ids.shape).astype(np.float32)
@@ -150,8 +153,28 @@ def test_prefill_block_sizes(dev, fmt, block, E, E2, H, I):
     x = synth.activations(rng, M, H)
     y_ref = oracle.experts.moe_layer("prefill", x, w, ids, bank, sh)
     y, y2 = (ops.experts_prefill(bf16_dev(x, dev), torch.from_numpy(w).to(dev), torch.from_numpy(ids).to(dev),
-                                 to_device_bank(bank, dev, slice(0, n)), to_device_bank(sh, dev)) for n in (E, E2))
+                                 to_device_bank(bank, dev, slice(0, r)), to_device_bank(sh, dev)) for r in (E, E2))
     assert torch.equal(y, y2)
     got = to_np(y).astype(np.float64)
     assert np.linalg.norm(got - y_ref) <= 1e-2 * np.linalg.norm(y_ref)
     assert cosine(got, y_ref) >= COS_TOL, cosine(got, y_ref)
+
+
+def test_prefill_bf16_beyond_2gib(dev):
+    """A bf16 call whose activations pass the 31-bit offsets of the LDS-DMA GEMM
+    takes the register-staged one: equal to the same tokens in two calls that
+    fit, within the rounding of bf16 sums taken in another order."""
+    M, k, E, H, I = 60000, 8, 16, 128, 2048
+    assert M * (k + 1) * I * 2 > 2**31 > M // 2 * (k + 1) * I * 2
+    g = torch.Generator(device=dev).manual_seed(3)
+    gu = (torch.randn((E, 2 * I, H), generator=g, device=dev) * 0.05).to(torch.bfloat16)
+    dn = (torch.randn((E, H, I), generator=g, device=dev) * 0.02).to(torch.bfloat16)
+    x = torch.randn((M, H), generator=g, device=dev).to(torch.bfloat16)
+    w, ids = ops.route_softmax_topk(torch.randn((M, E), generator=g, device=dev), k, True)
+    bank = ops.ExpertBank("bf16", gu, dn)
+    y = ops.experts_prefill(x, w, ids, bank)
+    h = M // 2
+    halves = torch.cat([ops.experts_prefill(x[s].contiguous(), w[s].contiguous(), ids[s].contiguous(), bank)
+                        for s in (slice(0, h), slice(h, M))])
+    err = (y.double() - halves.double()).norm() / halves.double().norm()
+    assert float(err) <= 4e-3  # one bf16 rounding (2^-9 relative) on each side
