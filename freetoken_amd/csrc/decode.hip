@@ -47,9 +47,9 @@ __device__ __forceinline__ size_t row_bytes(int K) {
 
 // K placement inside a 128-wide K block: MFMA j (0..3) of lane group g = l/16
 // takes the 8 values starting at
-//   BF16   32j + 8g                 weights and activations: 16-byte pieces
-//                                   at 64j + 16g, one whole 64-byte line of a
-//                                   row per load instruction
+//   BF16   32j + 8g                 weights (from LDS) and activations: 16-byte
+//                                   pieces at 64j + 16g; a step holds j = 0, 1
+//                                   or 2, 3 of the block
 //   FP8    64(j/2) + 16g + 8(j%2)   weights (from LDS, see dma_compute): the
 //                                   16 bytes at 64i + 16g feed MFMAs 2i, 2i+1;
 //                                   activations: 128(j/2) + 32g + 16(j%2)
@@ -76,10 +76,6 @@ constexpr uint32_t b_piece_bytes(int j) {
 template <int FMT>
 struct RawA;
 template <>
-struct RawA<FMT_BF16> {
-  bf16x8 v[4];
-};
-template <>
 struct RawA<FMT_FP8> {
   u32x4 v[2];
 };
@@ -101,24 +97,15 @@ struct RawA<FMT_MXFP4> {
 template <int FMT>
 __device__ __forceinline__ void load_raw(__amdgpu_buffer_rsrc_t wr, __amdgpu_buffer_rsrc_t sr, uint32_t voff,
                                          uint32_t coff, int kb, uint32_t dead, RawA<FMT>& r) {
-  if constexpr (FMT == FMT_BF16) {
-    const uint32_t so = static_cast<uint32_t>(kb) * 256;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) r.v[j] = __builtin_bit_cast(bf16x8, buf_x4(wr, (voff | dead) + 64 * j, so));
-  } else {
-    static_assert(FMT == FMT_MXFP4, "FP8 weights take the LDS path (gemv_tile_dma)");
-    r.v[0] = buf_x4(wr, voff | dead, static_cast<uint32_t>(kb) * 64);
-    r.code = buf_u8(sr, coff | dead, static_cast<uint32_t>(kb) * 4);
-  }
+  static_assert(FMT == FMT_MXFP4, "the other formats take the LDS path (gemv_tile_dma)");
+  r.v[0] = buf_x4(wr, voff | dead, static_cast<uint32_t>(kb) * 64);
+  r.code = buf_u8(sr, coff | dead, static_cast<uint32_t>(kb) * 4);
 }
 
 // Dequantises raw bytes into four bf16x8 MFMA operands (exact conversions).
 template <int FMT>
 __device__ __forceinline__ void dequant(const RawA<FMT>& r, bf16x8 (&a)[4]) {
-  if constexpr (FMT == FMT_BF16) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) a[j] = r.v[j];
-  } else if constexpr (FMT == FMT_FP8) {
+  if constexpr (FMT == FMT_FP8) {
     const uint32_t wds[8] = {r.v[0][0], r.v[0][1], r.v[0][2], r.v[0][3], r.v[1][0], r.v[1][1], r.v[1][2], r.v[1][3]};
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -147,7 +134,6 @@ template <int FMT, int NMAT, int NCH>
 struct KStage {
   RawA<FMT> w[NMAT];
   u32x4 b[NCH][4];
-  float sc[NMAT];  // FP8: the 128x128 block scale of each tile for this K block
 };
 
 // Lanes whose route column lies past the segment's end carry kOutOfRange and
@@ -170,12 +156,6 @@ __device__ __forceinline__ void load_stage(KStage<FMT, NMAT, NCH>& st, const WTi
                                            uint32_t dead) {
 #pragma unroll
   for (int m = 0; m < NMAT; ++m) load_raw<FMT>(wt.wr, wt.sr, wt.wvoff[m], wt.soff[m], kb, dead, st.w[m]);
-  if constexpr (FMT == FMT_FP8) {
-    // wave-uniform address: one request per tile, in flight with the weights
-#pragma unroll
-    for (int m = 0; m < NMAT; ++m)
-      st.sc[m] = buf_f32(wt.sr, wt.soff[m] | dead, static_cast<uint32_t>(kb) * 4);
-  }
   const uint32_t so = static_cast<uint32_t>(kb) * 256;
 #pragma unroll
   for (int c = 0; c < NCH; ++c)
@@ -185,31 +165,16 @@ __device__ __forceinline__ void load_stage(KStage<FMT, NMAT, NCH>& st, const WTi
 
 template <int FMT, int NMAT, int NCH>
 __device__ __forceinline__ void compute_stage(const KStage<FMT, NMAT, NCH>& st, f32x4 (&acc)[NMAT][NCH]) {
-  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int m = 0; m < NMAT; ++m) {
     bf16x8 a[4];
-    if constexpr (FMT == FMT_BF16) {
+    dequant<FMT>(st.w[m], a);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) a[j] = st.w[m].v[j];  // element-wise: no aggregate copy
-    } else {
-      dequant<FMT>(st.w[m], a);
-    }
+    for (int c = 0; c < NCH; ++c)
 #pragma unroll
-    for (int c = 0; c < NCH; ++c) {
-      if constexpr (FMT == FMT_FP8) {
-        f32x4 t = zero;
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[j], __builtin_bit_cast(bf16x8, st.b[c][j]), t, 0, 0, 0);
-        acc[m][c] += t * st.sc[m];
-      } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          acc[m][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[j], __builtin_bit_cast(bf16x8, st.b[c][j]), acc[m][c],
-                                                              0, 0, 0);
-      }
-    }
+      for (int j = 0; j < 4; ++j)
+        acc[m][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[j], __builtin_bit_cast(bf16x8, st.b[c][j]), acc[m][c],
+                                                            0, 0, 0);
   }
 }
 
@@ -218,7 +183,7 @@ __device__ __forceinline__ void compute_stage(const KStage<FMT, NMAT, NCH>& st, 
 // and NCH activation chunks), between 2 and 4.
 template <int FMT, int NMAT, int NCH>
 constexpr int pipeline_depth() {
-  constexpr int wregs = FMT == FMT_BF16 ? 16 : FMT == FMT_FP8 ? 8 : 4;
+  constexpr int wregs = 4;
   constexpr int per_stage = NMAT * (wregs + 1) + NCH * 16;
   constexpr int fit = (200 - NMAT * NCH * 4 - 24) / per_stage;
   return fit < 2 ? 2 : fit > 4 ? 4 : fit;
@@ -265,35 +230,43 @@ __device__ __forceinline__ void gemv_tile(const WTiles<NMAT>& wt, int K, int kw,
     if (i + s < n) compute_stage(st[s], acc);
 }
 
-// Quantised weights (FP8, MXFP4) stream through LDS instead of registers.  A
-// register load instruction can cover at most 64 bytes of a row (4 lanes of
-// 16 bytes share a row in the MFMA operand layout), so the two halves of each
-// 128-byte line are fetched by different instructions and the line has to
-// stay in L2 between them.  A DMA instruction (buffer load to LDS) is free to
-// give its 64 lanes 8 whole rows: each fetches complete lines, which lets the
-// weights use the nontemporal policy (measured on MI355X: 7.1 TB/s against
-// 6.2 TB/s for the default policy on a plain stream).  A K step covers 128
-// bytes of every row: one K block of FP8, two of MXFP4.  Each wave owns a ring
-// of stages in LDS (dma_depth); a stage holds NMAT tiles of 16 rows x 128
-// bytes.  Chunk c (16 bytes) of tile row r lands at slot c ^ (r & 7) of the
-// row, spreading the operand reads over the LDS banks.  A lane's operands are
-// chunks g and 4 + g of its row: FP8 values 16g.. and 64 + 16g.. of the K
-// block (MFMAs 0, 1 and 2, 3); MXFP4 values 32g.. of the first and of the
-// second K block of the step.
+// Weights stream through LDS instead of registers (the register ring above is
+// left for MXFP4 with K not a multiple of 256).  A register load instruction can
+// cover at most 64 bytes of a row (4 lanes of 16 bytes share a row in the MFMA
+// operand layout), so the two halves of each 128-byte line are fetched by
+// different instructions and the line has to stay in L2 between them.  A DMA
+// instruction (buffer load to LDS) is free to give its 64 lanes 8 whole rows:
+// each fetches complete lines, which lets the weights use the nontemporal policy
+// (measured on MI355X: 7.1 TB/s against 6.2 TB/s for the default policy on a
+// plain stream; bf16 experts, register loads -> LDS, H 2048, I 768, 128 experts,
+// top-8: 4 tokens 71.7 -> 61.4 us, 24 196 -> 170, 64 233 -> 201, 256 318 -> 227;
+// a bf16 shared expert beside MXFP4 at 64 tokens, H 5120, 247 -> 235).
+// A K step covers 128 bytes of every row: one K block of FP8, two of MXFP4, half
+// a block of bf16.  Each wave owns a ring of stages in LDS (dma_depth); a stage
+// holds NMAT tiles of 16 rows x 128 bytes.  Chunk c (16 bytes) of tile row r
+// lands at slot c ^ (r & 7) of the row, spreading the operand reads over the LDS
+// banks.  A lane's operands are chunks g and 4 + g of its row: FP8 values 16g..
+// and 64 + 16g.. of the K block (MFMAs 0, 1 and 2, 3); bf16 values 8g.. and
+// 32 + 8g.. of the step (one MFMA each); MXFP4 values 32g.. of the first and of
+// the second K block of the step.
 constexpr int kTileBytes = 16 * 128;
 constexpr int kNtPolicy = 2;  // cache policy bits of a nontemporal load
 
 template <int FMT>
 constexpr int dma_kstep() {  // K values per step
-  return FMT == FMT_FP8 ? 128 : 256;
+  return FMT == FMT_BF16 ? 64 : FMT == FMT_FP8 ? 128 : 256;
 }
 template <int FMT>
 constexpr int dma_pieces() {  // activation loads (16 bytes) per chunk and step
-  return FMT == FMT_FP8 ? 4 : 8;
+  return FMT == FMT_BF16 ? 2 : FMT == FMT_FP8 ? 4 : 8;
+}
+template <int FMT, bool HELD = false>
+constexpr int dma_weight_ops() {  // vector memory instructions per tile and step (HELD: no per-step scale load)
+  return FMT == FMT_BF16 || HELD ? 2 : 3;
 }
 template <int FMT, int NMAT, int NCH, bool CT = false>
 constexpr int dma_per_step() {  // vector memory instructions of one dma_issue (CT: codes from the LDS table)
-  return (CT ? 2 : 3) * NMAT + dma_pieces<FMT>() * NCH;
+  return dma_weight_ops<FMT, CT>() * NMAT + dma_pieces<FMT>() * NCH;
 }
 
 // Per-step side data of a tile: FP8 the 128x128 block scale (wave-uniform);
@@ -301,6 +274,8 @@ constexpr int dma_per_step() {  // vector memory instructions of one dma_issue (
 // each word is the lane group's code).
 template <int FMT>
 struct DmaSide;
+template <>
+struct DmaSide<FMT_BF16> {};
 template <>
 struct DmaSide<FMT_FP8> {
   float s;
@@ -344,7 +319,7 @@ __device__ __forceinline__ void dma_issue(const DmaTiles<NMAT>& dt, __amdgpu_buf
     for (int m = 0; m < NMAT; ++m) {
       if constexpr (FMT == FMT_FP8)
         side[m].s = buf_f32(dt.sr, dt.soff[m] | dead, static_cast<uint32_t>(step) * 4);
-      else
+      else if constexpr (FMT == FMT_MXFP4)
         side[m].codes = buf_x2(dt.sr, dt.soff[m] | dead, static_cast<uint32_t>(step) * 8);
     }
   }
@@ -353,7 +328,7 @@ __device__ __forceinline__ void dma_issue(const DmaTiles<NMAT>& dt, __amdgpu_buf
   for (int c = 0; c < NCH; ++c)
 #pragma unroll
     for (int j = 0; j < dma_pieces<FMT>(); ++j) {
-      const uint32_t piece = FMT == FMT_FP8 ? b_piece_bytes<FMT_FP8>(j) : 256 * (j >> 2) + b_piece_bytes<FMT_MXFP4>(j & 3);
+      const uint32_t piece = FMT == FMT_MXFP4 ? 256 * (j >> 2) + b_piece_bytes<FMT_MXFP4>(j & 3) : b_piece_bytes<FMT>(j);
       b[c][j] = buf_x4(br, (bvoff[c] | dead) + piece, sb);
     }
 }
@@ -384,7 +359,15 @@ __device__ __forceinline__ void dma_compute(const uint8_t* stage, uint32_t rd0, 
   }
 #pragma unroll
   for (int m = 0; m < NMAT; ++m) {
-    if constexpr (FMT == FMT_FP8) {
+    if constexpr (FMT == FMT_BF16) {
+#pragma unroll
+      for (int c = 0; c < NCH; ++c) {
+        acc[m][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w0[m]),
+                                                            __builtin_bit_cast(bf16x8, b[c][0]), acc[m][c], 0, 0, 0);
+        acc[m][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w1[m]),
+                                                            __builtin_bit_cast(bf16x8, b[c][1]), acc[m][c], 0, 0, 0);
+      }
+    } else if constexpr (FMT == FMT_FP8) {
       RawA<FMT_FP8> r;
       r.v[0] = w0[m];
       r.v[1] = w1[m];
@@ -591,8 +574,22 @@ constexpr int act_col_bytes() {
   return dma_kstep<FMT>() * 2;
 }
 template <int FMT>
-constexpr int act_copies() {  // 1 KB copies per wave per chunk and step
-  return 16 * act_col_bytes<FMT>() / 1024 / kDecWaves;
+constexpr int act_copies() {  // 1 KB copies per wave per chunk and step (bf16: see act_ops)
+  return FMT == FMT_BF16 ? 1 : 16 * act_col_bytes<FMT>() / 1024 / kDecWaves;
+}
+// Activation copies of a step per wave.  A bf16 chunk is two copies: with two
+// chunks every wave has one, with one chunk waves 2 and 3 repeat those of 0 and
+// 1 (the same bytes), so that every wave issues the same number.
+template <int FMT, int NCH>
+constexpr int act_ops() {
+  return FMT == FMT_BF16 ? 1 : NCH * act_copies<FMT>();
+}
+// Slot position of 16-byte piece p of column c: the 16 columns of one operand
+// read hit distinct banks (a bf16 column is 8 pieces: two columns span the
+// banks).
+template <int FMT>
+__device__ __forceinline__ int act_piece_pos(int p, int c) {
+  return FMT == FMT_BF16 ? p ^ ((c >> 1) & 7) : p ^ c;
 }
 template <int FMT, int NCH>
 constexpr int act_slot_bytes() {
@@ -600,7 +597,7 @@ constexpr int act_slot_bytes() {
 }
 template <int FMT, int NMAT, int NCH, bool CR = false>
 constexpr int sh_per_step() {  // vector memory instructions of one sh_issue (CR: codes in registers)
-  return (CR ? 2 : 3) * NMAT + NCH * act_copies<FMT>();
+  return dma_weight_ops<FMT, CR>() * NMAT + act_ops<FMT, NCH>();
 }
 template <int FMT, int NMAT, int CMAX>
 constexpr int sh_act_ring_bytes() {  // the larger of the NCH variants up to CMAX chunks per pass (4: wide kernels)
@@ -627,9 +624,14 @@ __device__ __forceinline__ void sh_issue(const DmaTiles<NMAT>& dt, __amdgpu_buff
     for (int m = 0; m < NMAT; ++m) {
       if constexpr (FMT == FMT_FP8)
         side[m].s = buf_f32(dt.sr, dt.soff[m] | dead, static_cast<uint32_t>(step) * 4);
-      else
+      else if constexpr (FMT == FMT_MXFP4)
         side[m].codes = buf_x2(dt.sr, dt.soff[m] | dead, static_cast<uint32_t>(step) * 8);
     }
+  }
+  if constexpr (FMT == FMT_BF16) {
+    const int q = NCH == 1 ? wave & 1 : wave;
+    lds_dma16_cached(br, aslot + q * 1024, avoff[0][0] | dead, static_cast<uint32_t>(step) * CB);
+    return;
   }
 #pragma unroll
   for (int c = 0; c < NCH; ++c)
@@ -651,8 +653,10 @@ __device__ __forceinline__ void sh_compute(const uint8_t* wstage, const uint8_t*
 #pragma unroll
     for (int j = 0; j < P; ++j) {
       // piece (16 bytes) of the lane's MFMA operand j, then its swizzled position
-      const int pp = FMT == FMT_FP8 ? 8 * (j >> 1) + 2 * g + (j & 1) : 16 * (j >> 2) + 4 * g + (j & 3);
-      b[c][j] = *reinterpret_cast<const u32x4*>(aslot + c * 16 * CB + r16 * CB + ((pp ^ r16) << 4));
+      const int pp = FMT == FMT_BF16  ? 4 * j + g
+                     : FMT == FMT_FP8 ? 8 * (j >> 1) + 2 * g + (j & 1)
+                                      : 16 * (j >> 2) + 4 * g + (j & 3);
+      b[c][j] = *reinterpret_cast<const u32x4*>(aslot + c * 16 * CB + r16 * CB + (act_piece_pos<FMT>(pp, r16) << 4));
     }
   dma_compute<FMT, NMAT, NCH>(wstage, rd0, rd1, 8 * g, b, side, acc);
 }
@@ -898,9 +902,8 @@ __device__ __forceinline__ void decode_pass(const DecodeArgs& a, const BankView&
   }
   f32x4 acc[NMAT][NCH];
   // FP8 always, MXFP4 when a K step (two K blocks) divides K: the LDS path
-  constexpr bool kDma = FMT == FMT_FP8 || FMT == FMT_MXFP4;
-  if (kDma && K % dma_kstep<FMT>() == 0) {
-    if constexpr (kDma) {
+  if (K % dma_kstep<FMT>() == 0) {
+    {
       DmaTiles<NMAT> dt;
       dt.wr = wt.wr;
       dt.sr = wt.sr;
@@ -910,7 +913,7 @@ __device__ __forceinline__ void decode_pass(const DecodeArgs& a, const BankView&
         const int tile_row = (STAGE == 0 && m >= RT) ? inter + wrow0 + 16 * (m - RT) : wrow0 + 16 * m;
 #pragma unroll
         for (int h = 0; h < 2; ++h) dt.voff[m][h] = static_cast<uint32_t>(tile_row + 8 * h + dr) * rb + dc * 16;
-        dt.soff[m] = FMT == FMT_FP8 ? wt.soff[m] : static_cast<uint32_t>(tile_row + r16) * (K / 32);
+        dt.soff[m] = FMT == FMT_MXFP4 ? static_cast<uint32_t>(tile_row + r16) * (K / 32) : wt.soff[m];
       }
       uint8_t* ring = smem + wave * dma_ring_bytes<FMT, NMAT, WIDE>();
       if constexpr (KS == 1) {
@@ -922,9 +925,11 @@ __device__ __forceinline__ void decode_pass(const DecodeArgs& a, const BankView&
         for (int c = 0; c < NCH; ++c)
 #pragma unroll
           for (int v = 0; v < act_copies<FMT>(); ++v) {
-            const int colc = (wave * act_copies<FMT>() + v) * (1024 / CB) + lane / (CB / 16);
-            const int piece = (lane % (CB / 16)) ^ colc;
-            const int col = base + c * 16 + colc;
+            // (bf16: copy q of the step covers 8 columns of chunk q / 2)
+            const int q = FMT == FMT_BF16 ? (NCH == 1 ? wave & 1 : wave) : wave * act_copies<FMT>() + v;
+            const int colc = (FMT == FMT_BF16 ? q & 1 : q) * (1024 / CB) + lane / (CB / 16);
+            const int piece = act_piece_pos<FMT>(lane % (CB / 16), colc);
+            const int col = base + (FMT == FMT_BF16 ? q >> 1 : c) * 16 + colc;
             if (col < sv.count) {
               int row;
               if (STAGE == 0) row = sv.shared ? sv.start + col : a.sorted[sv.start + col] / a.k;
@@ -953,7 +958,7 @@ __device__ __forceinline__ void decode_pass(const DecodeArgs& a, const BankView&
       }
     }
   } else {
-    if constexpr (FMT != FMT_FP8)  // FP8 K is a multiple of 128: never here
+    if constexpr (FMT == FMT_MXFP4)  // the others' steps divide every K (a multiple of 128)
       gemv_tile<FMT, NMAT, NCH, KS>(wt, K, kw, br, bvoff, acc);
   }
 
@@ -967,7 +972,7 @@ __device__ __forceinline__ void decode_pass(const DecodeArgs& a, const BankView&
           tile_epilogue<STAGE>(a, sv, cd[c], wrow0 + 16 * t + g * 4, acc[t][c], acc[STAGE == 0 ? RT + t : t][c]);
       }
   } else {
-    if constexpr (kDma) __syncthreads();  // red overlays the waves' LDS rings
+    __syncthreads();  // red overlays the waves' LDS rings
 #pragma unroll
     for (int m = 0; m < NMAT; ++m)
 #pragma unroll
@@ -1004,8 +1009,7 @@ template <int FMT, int STAGE, int RT, int KS, int WIDE = 0>
 constexpr int chunks_per_pass() {
   if constexpr (WIDE && KS == 1 && FMT == FMT_FP8) return 4;
   if constexpr (KS == 1 && FMT == FMT_MXFP4) return 1;
-  if constexpr (STAGE == 0) return RT == 1 ? 2 : (FMT == FMT_BF16 ? 1 : 2);
-  return 2;
+    return 2;
 }
 
 template <int FMT, int STAGE, int RT, int KS, int WIDE = 0, bool CW = false>
@@ -1022,8 +1026,9 @@ __device__ __forceinline__ void decode_segment(const DecodeArgs& a, const BankVi
     } else if constexpr (CMAX == 1) {
       decode_pass<FMT, STAGE, RT, KS, 1>(a, bank, sv, base, row0, inter, smem, aring);
     } else {
-      if (sv.count - base <= 16) decode_pass<FMT, STAGE, RT, KS, 1, 0, CW>(a, bank, sv, base, row0, inter, smem, aring);
-      else decode_pass<FMT, STAGE, RT, KS, 2, 0, CW>(a, bank, sv, base, row0, inter, smem, aring);
+      constexpr int W = KS == 1 ? WIDE : 0;  // (bf16 beside wide FP8: two stages, as the ring is laid out)
+      if (sv.count - base <= 16) decode_pass<FMT, STAGE, RT, KS, 1, W, CW>(a, bank, sv, base, row0, inter, smem, aring);
+      else decode_pass<FMT, STAGE, RT, KS, 2, W, CW>(a, bank, sv, base, row0, inter, smem, aring);
     }
   }
 }
@@ -1042,7 +1047,9 @@ struct StageSmem {
       (FMT_R == FMT_FP8 || FMT_S == FMT_FP8) ? dma_ring_bytes<FMT_FP8, kNmat, WIDE && KS == 1>() : 0;
   static constexpr int kRingF4 =
       (FMT_R == FMT_MXFP4 || FMT_S == FMT_MXFP4) ? dma_ring_bytes<FMT_MXFP4, kNmat>() : 0;
-  static constexpr int kRing = kDecWaves * (kRingF8 > kRingF4 ? kRingF8 : kRingF4);
+  static constexpr int kRingBf = (FMT_R == FMT_BF16 || FMT_S == FMT_BF16) ? dma_ring_bytes<FMT_BF16, kNmat, WIDE && KS == 1>() : 0;
+  static constexpr int kRingQ = kRingF8 > kRingF4 ? kRingF8 : kRingF4;
+  static constexpr int kRing = kDecWaves * (kRingQ > kRingBf ? kRingQ : kRingBf);
   // without a K split the activation ring shared by the waves follows the waves' weight rings
   static constexpr bool kShAct = KS == 1;
   static constexpr int kActF8 = kShAct && (FMT_R == FMT_FP8 || FMT_S == FMT_FP8)
@@ -1052,7 +1059,12 @@ struct StageSmem {
       kShAct && (FMT_R == FMT_MXFP4 || FMT_S == FMT_MXFP4)
           ? sh_act_ring_bytes<FMT_MXFP4, kNmat, chunks_per_pass<FMT_MXFP4, STAGE, RT, KS>()>()
           : 0;
-  static constexpr int kAct = kActF8 > kActF4 ? kActF8 : kActF4;
+  static constexpr int kActBf =
+      kShAct && (FMT_R == FMT_BF16 || FMT_S == FMT_BF16)
+          ? sh_act_ring_bytes<FMT_BF16, kNmat, chunks_per_pass<FMT_BF16, STAGE, RT, KS>()>()
+          : 0;
+  static constexpr int kActQ = kActF8 > kActF4 ? kActF8 : kActF4;
+  static constexpr int kAct = kActQ > kActBf ? kActQ : kActBf;
   // MXFP4 with a K split: the e8m0 code table of the workgroup's tiles
   static constexpr int kCodes = (KS == kDecWaves && (FMT_R == FMT_MXFP4 || FMT_S == FMT_MXFP4)) ? kCodeTableBytes : 0;
   static constexpr int kRed = KS > 1 ? kRedFloats4 * 16 : 0;
@@ -1096,8 +1108,13 @@ __device__ __forceinline__ void decode_stage_block(const DecodeArgs& a, int bx, 
   }
   const int fmt = sv.shared ? FMT_S : FMT_R;
   if (fmt == FMT_BF16) {
-    if constexpr (FMT_R == FMT_BF16 || FMT_S == FMT_BF16)
-      decode_segment<FMT_BF16, STAGE, RT, KS>(a, bank, sv, row0, inter, smem, smem + kRing);
+    if constexpr (FMT_R == FMT_BF16 || FMT_S == FMT_BF16) {
+      // (cached: as for FP8 below)
+      if (sv.shared && a.M > a.seg_cap)
+        decode_segment<FMT_BF16, STAGE, RT, KS, WIDE, true>(a, bank, sv, row0, inter, smem, smem + kRing);
+      else
+        decode_segment<FMT_BF16, STAGE, RT, KS, WIDE>(a, bank, sv, row0, inter, smem, smem + kRing);
+    }
   } else if (fmt == FMT_FP8) {
     if constexpr (FMT_R == FMT_FP8 || FMT_S == FMT_FP8)
     {
@@ -1348,22 +1365,24 @@ static hipError_t launch_stage_t(int stage, const DecodeArgs& a, bool has_shared
       // share the activation chunks through LDS (half the activation reads
       // per weight byte of the RT = 2 K-split grid); measured C4 b=128 326 ->
       // 302 us, b=16-64 unchanged, b=8 slower (its grid no longer fills the
-      // GPU); MXFP4 (one chunk per pass) slower at b=8-64.  From 80 tokens
+      // GPU); MXFP4 (one chunk per pass) slower at b=8-64, bf16 8-13% slower at
+      // b=80-256 (its steps hold half the K).  From 80 tokens
       // (interleaved A/B against the K split): C4 b=80 471 -> 464 us, b=96
       // 480 -> 470, b=112 498 -> 478; b=32-64 equal within 2 us
       constexpr auto ks = decode_stage_kernel<FR, FS, 0, 1, 1>;
       return launch_one<ks>(dim3((imax + 63) / 64, gy), a, stream);
     }
     const dim3 g1((imax + 15) / 16, gy), g2((imax + 31) / 32, gy);
-    // FP8 calls of up to four tokens, or whose RT = 2 grid is a single round
+    // FP8 and bf16 calls of up to four tokens, or whose RT = 2 grid is a single round
     // of resident workgroups: few experts, many of the grid's segments empty
     // (routes to experts outside the slot bank), and the RT = 1 grid's twice
     // as many, half as long workgroups end together more evenly (C4 b=1
     // 72.5-72.8 -> 69.6-70.6 us, b=2 115.4-116.1 -> 109.7-109.8 us; b=4
     // 160.1 -> 156.7 and 176.9 -> 175.7 us on two boxes, b=3 equal; up to 8
     // tokens C2 b=8 was 5% slower; MXFP4 at C3 b=1 0.8 us slower, so it
-    // keeps RT = 2)
-    if (FR == FMT_FP8 &&
+    // keeps RT = 2; bf16 H 1024, I 512, 16 experts, top-2: 4 tokens 24.1 ->
+    // 22.7 us, H 4096, I 1536, 32 experts, top-8: 4 tokens 140.6 -> 138.5)
+    if ((FR == FMT_FP8 || FR == FMT_BF16) &&
         (a.M <= 4 ||
          static_cast<long long>(g2.x) * g2.y <= static_cast<long long>(cu_count()) * resident_per_cu<k2>()))
       return launch_one<k1>(g1, a, stream);
@@ -1382,10 +1401,11 @@ static hipError_t launch_stage_t(int stage, const DecodeArgs& a, bool has_shared
   // on the routed segments fill the GPU and one tile per wave is slower)
   const bool heavy_shared = has_shared && bytes_per_weight_x2(FS) >= 4 * bytes_per_weight_x2(FR);
   if (heavy_shared && a.M <= 2) return launch_one<k1>(g1, a, stream);
-  // one FP8 token: K split two ways (half the rows per workgroup's row group
+  // one FP8 or bf16 token: K split two ways (half the rows per workgroup's row group
   // walk, twice the workgroups); interleaved A/B: C4 b=1 69.6 -> 68.9 us, C2
-  // b=1 30.2 -> 29.3 us; from two tokens equal or slower
-  if (FR == FMT_FP8 && a.M == 1) {
+  // b=1 30.2 -> 29.3 us; bf16 H 2048, I 768 32.3 -> 30.7, H 1024, I 512 22.8 ->
+  // 20.6; from two tokens equal or slower
+  if ((FR == FMT_FP8 || FR == FMT_BF16) && a.M == 1) {
     constexpr auto kh = decode_stage_kernel<FR, FS, 1, 2, 2>;
     return launch_one<kh>(dim3(a.H / 64, gy), a, stream);
   }

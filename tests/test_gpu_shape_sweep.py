@@ -66,6 +66,31 @@ def test_decode_shape_sweep(dev, i):
     assert cosine(got, y_ref) >= COS_TOL, (case, cosine(got, y_ref))
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt,sfmt,E,H,I,sI,k,M", [
+    # bf16 through the LDS rings: 1 to 3 steps of 64 K per wave, one and two
+    # route chunks per pass, several shared pieces (cached weights)
+    ("bf16", None, 3, 128, 128, 0, 2, 1),
+    ("bf16", "bf16", 4, 384, 640, 384, 2, 40),
+    ("bf16", "bf16", 2, 1152, 128, 128, 2, 70),
+    # ... as the shared expert of the wide FP8 kernels and beside MXFP4
+    ("fp8", "bf16", 5, 384, 256, 384, 4, 150),
+    ("mxfp4", "bf16", 5, 512, 256, 128, 4, 33),
+])
+def test_decode_bf16_rings(dev, fmt, sfmt, E, H, I, sI, k, M):
+    rng = np.random.default_rng(H + I + M)
+    bank = synth.make_bank(fmt, E, H, I, rng)
+    shared = synth.make_bank(sfmt, 1, H, sI, rng) if sfmt else None
+    x = synth.activations(rng, M, H)
+    ids = _ids(rng, M, E, k)
+    w = rng.random((M, k), dtype=np.float32) + 0.05
+    y_ref = oracle.experts.moe_layer("decode", x, w, ids, bank, shared)
+    got = to_np(ops.experts_decode(bf16_dev(x, dev), torch.from_numpy(w).to(dev), torch.from_numpy(ids).to(dev),
+                                   to_device_bank(bank, dev), to_device_bank(shared, dev) if shared else None))
+    assert max_rel(got, y_ref) <= MAX_REL_TOL, max_rel(got, y_ref)
+    assert cosine(got, y_ref) >= COS_TOL, cosine(got, y_ref)
+
+
 def _prefill_config(i: int):
     rng = np.random.default_rng(8000 + i)
     fmt = ("fp8", "mxfp4", "bf16")[i % 3]
