@@ -1009,7 +1009,7 @@ template <int FMT, int STAGE, int RT, int KS, int WIDE = 0>
 constexpr int chunks_per_pass() {
   if constexpr (WIDE && KS == 1 && FMT == FMT_FP8) return 4;
   if constexpr (KS == 1 && FMT == FMT_MXFP4) return 1;
-    return 2;
+  return 2;
 }
 
 template <int FMT, int STAGE, int RT, int KS, int WIDE = 0, bool CW = false>

@@ -131,7 +131,7 @@ struct PrefillGemmArgs {
   int num_experts;          // bank rows taking part
   int numel;                // M * k
   int M, k;
-  uint32_t k_magic;         // ceil(2^32 / k), 0 for k = 1: r / k = umulhi(r, k_magic) for r < 2^26
+  uint32_t k_magic;         // ceil(2^32 / k), 0 for k = 1: umulhi(r, k_magic) is r / k or one more
   int block;                // routes per M block (BM)
   int wide;                 // bf16: an operand beyond 2 GiB (prefill_operands_fit is false)
   int max_blocks;           // routed M blocks of the grid

@@ -649,7 +649,15 @@ __global__ void __launch_bounds__(kQThreads) prefill_qgemm_kernel(PrefillGemmArg
     const int lim = col_limit(t);
     const uint32_t magic = !t.shared && a.x_token_rows ? a.k_magic : 0u;
     const int add = t.shared && !a.x_token_rows ? a.numel : 0;
-    auto row_of = [&](int r) -> uint32_t { return (magic ? __umulhi(static_cast<uint32_t>(r), magic) : static_cast<uint32_t>(r)) + add; };
+    auto row_of = [&](int r) -> uint32_t {
+      uint32_t q = static_cast<uint32_t>(r);
+      if (magic) {
+        q = __umulhi(q, magic);
+        // the rounded-up reciprocal gives at most one too many, from r = 2^32 / k on
+        q -= q * static_cast<uint32_t>(a.k) > static_cast<uint32_t>(r) ? 1u : 0u;
+      }
+      return q + add;
+    };
     const int ln = fresh_lane();
     if (kQuant && wave >= 4 && wave < 4 + BM / 64) {
       const int r = s_route[b][64 * (wave - 4) + ln];

@@ -178,3 +178,21 @@ def test_prefill_bf16_beyond_2gib(dev):
                         for s in (slice(0, h), slice(h, M))])
     err = (y.double() - halves.double()).norm() / halves.double().norm()
     assert float(err) <= 4e-3  # one bf16 rounding (2^-9 relative) on each side
+
+
+@pytest.mark.parametrize("fmt", ["fp8", "bf16"])
+def test_prefill_token_of_route_many_choices(dev, fmt):
+    """The token of a route (route / k) where k times the route index passes
+    2^32: k = 4369 divides 2^32 - 1, so a rounded-up 32-bit reciprocal is one
+    too large for the last choice of every token from 225 on.  Only the last
+    choice has weight: the sums hold one term and equal a top-1 call's."""
+    M, k, H, I = 320, 4369, 128, 128
+    rng = np.random.default_rng(11)
+    bank = to_device_bank(synth.make_bank(fmt, 4, H, I, rng), dev)
+    x = bf16_dev(synth.activations(rng, M, H), dev)
+    ids = torch.from_numpy(rng.integers(0, 4, size=(M, k)).astype(np.int32)).to(dev)
+    w = torch.zeros((M, k), device=dev)
+    w[:, -1] = 1.0
+    y = ops.experts_prefill(x, w, ids, bank)
+    y1 = ops.experts_prefill(x, w[:, -1:].contiguous(), ids[:, -1:].contiguous(), bank)
+    assert torch.equal(y, y1)
