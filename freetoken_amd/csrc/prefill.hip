@@ -891,8 +891,9 @@ __global__ void __launch_bounds__(kQThreads) prefill_qgemm_kernel(PrefillGemmArg
                 uu = fminf(fmaxf(uu, -lim), lim);
               }
               float act;
-              if constexpr (decltype(kind)::value == ACT_SILU) act = act_fixed<ACT_SILU>(gg);
-              else act = act_apply(a.act_kind, gg);
+              if constexpr (decltype(kind)::value != ACT_SILU) act = act_apply(a.act_kind, gg);
+              else if constexpr (kQuant) act = act_fixed<ACT_SILU>(gg);
+              else act = act_apply(ACT_SILU, gg);  // divides, as the decode does
               o[v4] = act * uu;
             }
 #pragma unroll

@@ -57,11 +57,13 @@ __device__ __forceinline__ float quant_value(float x, float s, float mul) {
   return fminf(fmaxf(y, -448.0f), 448.0f);
 }
 
-// Activation with its kind fixed at compile time, for epilogues that hoist
-// the runtime choice out of their per-value loops.  SiLU multiplies by the
-// hardware reciprocal (within 1 ulp) instead of dividing: its result is
-// rounded to bf16 next, and the exponential is the hardware one either way,
-// so the IEEE division bought no exactness (the other kinds are act_apply).
+// Activation of the quantised formats' epilogues, which hoist the runtime
+// choice of its kind out of their per-value loops.  SiLU multiplies by the
+// hardware reciprocal (within 1 ulp) instead of dividing: its product with the
+// up value is rounded to bf16 and then to e4m3, and the exponential is the
+// hardware one either way.  Below gates of about -87.3 the reciprocal is
+// subnormal and comes out as 0, which bf16 outputs would show: the bf16
+// epilogue divides (the other kinds are act_apply).
 template <int ACT>
 __device__ __forceinline__ float act_fixed(float g) {
   if constexpr (ACT == ACT_SILU) return g * __builtin_amdgcn_rcpf(1.0f + __expf(-g));

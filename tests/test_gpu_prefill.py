@@ -196,3 +196,27 @@ def test_prefill_token_of_route_many_choices(dev, fmt):
     y = ops.experts_prefill(x, w, ids, bank)
     y1 = ops.experts_prefill(x, w[:, -1:].contiguous(), ids[:, -1:].contiguous(), bank)
     assert torch.equal(y, y1)
+
+
+def test_prefill_bf16_silu_is_the_decode_one(dev):
+    """bf16 SwiGLU over gates of -88.5 to 88.5, where the reciprocal of
+    1 + exp(-gate) passes from subnormal to 1: the products of every weight with
+    a one or a zero are exact, so prefill and decode give the same bits, and the
+    64-bit value within one bf16 rounding (8 significant bits: 2^-8) on top of
+    the exponential's (its argument, up to 88, rounded to 24 bits)."""
+    n, M = 1024, 12
+    gate = torch.linspace(-88.5, 88.5, n).to(torch.bfloat16)
+    gu = torch.zeros((1, 2 * n, n), dtype=torch.bfloat16)
+    gu[0, :n, 0] = gate
+    gu[0, n:, 1] = 1.0
+    x = torch.zeros((M, n), dtype=torch.bfloat16)
+    x[:, 0] = 1.0
+    x[:, 1] = 2.0 ** torch.arange(0, 10 * M, 10)  # the up values: large enough for the smallest products to be normal
+    bank = ops.ExpertBank("bf16", gu.to(dev), torch.eye(n, dtype=torch.bfloat16)[None].to(dev))
+    args = (x.to(dev), torch.ones((M, 1), device=dev), torch.zeros((M, 1), dtype=torch.int32, device=dev), bank)
+    y, yd = ops.experts_prefill(*args).cpu(), ops.experts_decode(*args).cpu()
+    assert torch.equal(y, yd)
+    g = gate.double()
+    ref = (g / (1 + torch.exp(-g)))[None, :] * x[:, 1:2].double()
+    seen = ref.abs() > 2.0 ** -120
+    assert float(((y.double() - ref).abs() / ref.abs())[seen].max()) <= 2.0 ** -8 + 88.5 * 2.0 ** -23
