@@ -24,11 +24,13 @@ def _ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 
 
-def _stream(device: torch.device) -> int:
-    # the raw handle of the current stream: torch.cuda.current_stream builds a Stream object
-    # on every call, 2 us of the 26 us that a small eager decode call takes on the host
-    index = device.index
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+def _stream(device) -> int:
+    # a tensor's device: the raw handle of its current stream (torch.cuda.current_stream builds a
+    # Stream object on every call, 2 us of the 26 us that a small eager decode call takes on the host)
+    if isinstance(device, torch.device) and device.type == "cuda" and device.index is not None:
+        return torch._C._cuda_getCurrentRawStream(device.index)
+    # None, an index, a name, or a device without an index
+    return torch.cuda.current_stream(device).cuda_stream
 
 
 def _require_gpu(*tensors: torch.Tensor) -> None:

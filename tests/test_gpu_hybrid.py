@@ -289,3 +289,34 @@ def test_flag_wait_unblocks_on_watchdog(dev):
     assert float(marker.item()) == 1.0 and not ex.healthy
     ex.hold(False)
     ex.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("side", [False, True])
+def test_executor_streams_of_every_device_form(dev, side):
+    """submit and wait take the current stream of a device given as nothing, an
+    index, a name or a torch.device, with and without an index; the CPU is
+    refused."""
+    from freetoken_amd import ops
+
+    rng = np.random.default_rng(103)
+    E, H, I, M, k = 4, 256, 128, 2, 2
+    hb = to_device_bank(synth.make_bank("bf16", E, H, I, rng), "cpu")
+    x = torch.from_numpy(synth.activations(rng, M, H)).to(torch.bfloat16).pin_memory()
+    w = torch.full((M, k), 0.5, dtype=torch.float32).pin_memory()
+    ids = torch.tensor([[0, 1], [2, 3]], dtype=torch.int32).pin_memory()
+    y = torch.zeros((M, H), dtype=torch.bfloat16).pin_memory()
+    ex = ops.CpuExecutor(threads=2, watchdog_s=5.0)
+    y_ref = ex.run(hb, x, w, ids)
+    with torch.cuda.stream(torch.cuda.Stream() if side else torch.cuda.current_stream()):
+        handle = torch.cuda.current_stream().cuda_stream
+        for form in ((), (None,), (0,), ("cuda",), ("cuda:0",), (torch.device("cuda"),), (torch.device("cuda", 0),)):
+            kw = {"device": form[0]} if form else {}
+            assert ops._stream(*(form or (None,))) == handle
+            y.zero_()
+            ex.wait(ex.submit(hb, x, w, ids, y, **kw), **kw)
+            torch.cuda.synchronize()
+            assert torch.equal(y, y_ref), form
+    with pytest.raises(ValueError):
+        ops._stream(torch.device("cpu"))
+    ex.close()

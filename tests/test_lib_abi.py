@@ -87,6 +87,26 @@ def test_ops_reject_cpu_tensors():
         ops.route_softmax_topk(torch.zeros(2, 8), 2, True)
 
 
+def test_stream_without_an_index_is_the_current_one(monkeypatch):
+    """Everything torch.cuda.current_stream takes goes to it, except a device
+    with an index, whose raw handle is read directly."""
+    import torch
+
+    from freetoken_amd import ops
+
+    asked = []
+
+    class Stream:
+        cuda_stream = 7
+
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: asked.append(device) or Stream())
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda index: 100 + index)
+    forms = [None, 1, "cuda", "cuda:1", torch.device("cuda"), torch.device("cpu", 0)]
+    assert [ops._stream(d) for d in forms] == [7] * len(forms)
+    assert asked == forms
+    assert ops._stream(torch.device("cuda", 3)) == 103
+
+
 def test_empty_batch_is_a_noop():
     """M = 0 (empty tensors, NULL data pointers) returns OK from every router
     and expert entry point without reading a pointer or launching; M < 0 is an
