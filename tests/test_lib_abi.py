@@ -78,6 +78,27 @@ def test_workspace_query():
     assert n >= (576 * 2048 + 512 * 7168 + 64 * 7168) * 2
 
 
+@pytest.mark.parametrize("fmt", [_lib.FMT_BF16, _lib.FMT_FP8_B128, _lib.FMT_MXFP4])
+def test_prefill_workspace_grows_with_the_batch(fmt):
+    """A workspace sized at the largest batch serves every smaller one, across
+    the changes of routes per tile and, for bf16, of the kernel at 2 GiB of an
+    operand."""
+    L = _lib.lib()
+
+    def sizes(rows, H, I, k, Ms):
+        bank = _lib.FtmoeBank(fmt, rows, H, I, 16, 16, 16, 16)
+        return [L.ftmoe_experts_prefill_workspace(M, k, ctypes.byref(bank), None) for M in Ms]
+
+    for rows, H, I, k in [(1023, 128, 128, 8), (600, 640, 128, 7), (16, 1152, 128, 2), (3, 128, 384, 1), (256, 256, 128, 8)]:
+        top = 340 * rows // k + 40
+        got = sizes(rows, H, I, k, range(1, top, max(1, top // 20000)))
+        assert got == sorted(got), (rows, H, I, k)
+    # one operand (routed activations, tokens) passes 2 GiB of bf16 values inside the range
+    for rows, H, I, k, M in [(1023, 128, 2048, 8, 58254), (16, 128, 2048, 8, 58254), (64, 7168, 128, 1, 149796)]:
+        got = sizes(rows, H, I, k, range(M - 50, M + 50))
+        assert got == sorted(got), (rows, H, I, k)
+
+
 def test_ops_reject_cpu_tensors():
     import torch
 
