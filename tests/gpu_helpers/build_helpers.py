@@ -8,7 +8,8 @@ from pathlib import Path
 
 HERE = Path(__file__).resolve().parent
 ROOT = HERE.parents[1]
-HELPERS = {"libbf16check.so": "bf16_rounding.hip", "libquantcheck.so": "quant_division.hip"}
+HELPERS = {"libbf16check.so": "bf16_rounding.hip", "libquantcheck.so": "quant_division.hip",
+           "libprefillblocks.so": "prefill_blocks.hip"}
 
 
 def build() -> list[Path]:

@@ -2,6 +2,9 @@
 
 from __future__ import annotations
 
+import ctypes
+from pathlib import Path
+
 import numpy as np
 import pytest
 import torch
@@ -9,12 +12,24 @@ import torch
 import oracle
 from oracle import synth
 from oracle.numerics import bf16_round
-from freetoken_amd import ops
+from freetoken_amd import _lib, ops
 
 from _helpers import bf16_dev, to_device_bank, to_np
 from conftest import COS_TOL, MAX_REL_TOL, cosine, max_rel
 
 pytestmark = pytest.mark.gpu
+
+BLOCKS_HELPER = Path(__file__).resolve().parent / "gpu_helpers" / "libprefillblocks.so"
+_FMT_CODE = {"bf16": _lib.FMT_BF16, "fp8": _lib.FMT_FP8_B128, "mxfp4": _lib.FMT_MXFP4}
+
+
+def _block(fmt, M, k, rows, H, I):
+    """Routes per tile of a prefill call (the launch's own rule)."""
+    if not BLOCKS_HELPER.exists():
+        from tests.gpu_helpers import build_helpers  # built by __graft_entry__.build(); rebuilt if absent
+
+        build_helpers.build()
+    return ctypes.CDLL(str(BLOCKS_HELPER)).prefill_blocks(_FMT_CODE[fmt], M, k, rows, H, I)
 
 
 @pytest.mark.parametrize("rows,K", [(1, 128), (37, 1024), (513, 7168)])
@@ -129,9 +144,9 @@ def test_prefill_activation_variants(dev, fmt, activation):
 
 @pytest.mark.parametrize("H,I", [(640, 384), (128, 1152), (1024, 128)])
 @pytest.mark.parametrize("fmt,block,n,E,E2", [
-    ("fp8", 64, 1, 16, 3), ("fp8", 128, 1, 4, 16), ("fp8", 256, 1, 4, 16),
-    ("mxfp4", 64, 1, 16, 3), ("mxfp4", 128, 1, 4, 16), ("mxfp4", 256, 1, 4, 16),
-    ("bf16", 64, 1, 16, 3), ("bf16", 128, 1, 4, 16), ("bf16", 256, 2, 3, 16),
+    ("fp8", 64, 2, 16, 3), ("fp8", 128, 1, 4, 16), ("fp8", 256, 1, 4, 16),
+    ("mxfp4", 64, 2, 16, 3), ("mxfp4", 128, 1, 4, 16), ("mxfp4", 256, 1, 4, 16),
+    ("bf16", 64, 2, 16, 3), ("bf16", 128, 1, 4, 16), ("bf16", 256, 2, 3, 16),
 ])
 def test_prefill_block_sizes(dev, fmt, block, n, E, E2, H, I):
     """Every routes-per-tile variant of the GEMMs at its edges: one expert with
@@ -144,10 +159,13 @@ def test_prefill_block_sizes(dev, fmt, block, n, E, E2, H, I):
     whose bf16 rounding, and with it its e4m3 code, falls the other way (the
     sums differ in their last bit) moves one output row by up to 1/16 of that
     product, which the maximum over few outputs would show as 2-3%."""
+    if fmt == "mxfp4" and block == 256:  # (those with a K of 1 mod 4 blocks take 128)
+        H, I = {640: (768, 384), 128: (256, 1408), 1024: (1024, 256)}[H]
     rng = np.random.default_rng(block + H)
     flat = np.repeat(np.arange(3, dtype=np.int32), [n * block, n * block + 1, 1])
     ids = rng.permutation(flat).reshape(-1, 2)
     M = ids.shape[0]
+    assert _block(fmt, M, 2, E, H, I) == block != _block(fmt, M, 2, E2, H, I)
     w = rng.uniform(0.1, 1.0, size=ids.shape).astype(np.float32)
     bank, sh = synth.make_bank(fmt, 16, H, I, rng), synth.make_bank(fmt, 1, H, I, rng)
     x = synth.activations(rng, M, H)
@@ -158,6 +176,103 @@ def test_prefill_block_sizes(dev, fmt, block, n, E, E2, H, I):
     got = to_np(y).astype(np.float64)
     assert np.linalg.norm(got - y_ref) <= 1e-2 * np.linalg.norm(y_ref)
     assert cosine(got, y_ref) >= COS_TOL, cosine(got, y_ref)
+
+
+def _bank_rows(bank, rows):
+    """The device bank's rows in turn, `rows` of them."""
+    def take(t):
+        idx = torch.arange(rows, device=bank.gate_up.device) % t.shape[0]
+        return t.view(torch.uint8)[idx].view(t.dtype)
+
+    return ops.ExpertBank(bank.fmt, *(take(t) if t is not None else None
+                                      for t in (bank.gate_up, bank.down, bank.gate_up_scale, bank.down_scale)))
+
+
+@pytest.mark.parametrize("hb,ib,shared", [(5, 1, True), (6, 2, False), (7, 3, True), (9, 4, False), (1, 6, True),
+                                          (2, 5, False), (3, 7, False), (4, 9, True)])
+@pytest.mark.parametrize("fmt", ["fp8", "mxfp4", "bf16"])
+def test_prefill_many_tiles_per_workgroup(dev, fmt, hb, ib, shared):
+    """The persistent GEMMs with several tiles for every workgroup, where copies,
+    scale groups, route lists and router weights run on from tile to tile: K of
+    1 to 9 blocks of 128 in both GEMMs (shorter than the copies run ahead, up to
+    twice that, every remainder of the groups of four).  One routing over 60
+    experts; more bank rows take a smaller tile, with the same bits; tokens taken
+    at random are held against the oracle (by the 2-norm, as above)."""
+    H, I, E, k = 128 * hb, 128 * ib, 60, 8
+    rng = np.random.default_rng(100 * hb + ib)
+    distinct = 7  # weights that repeat over the bank's rows: no neighbour has its expert's
+    bank, sh = synth.make_bank(fmt, distinct, H, I, rng), synth.make_bank(fmt, 1, H, I, rng) if shared else None
+    M = 330 * E // k
+    x = synth.activations(rng, M, H)
+    w, ids = oracle.routing.softmax_topk(synth.normal(rng, (M, E)), k, True)
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    counts = np.bincount(ids.ravel(), minlength=E)
+    dbank, dsh = to_device_bank(bank, dev), to_device_bank(sh, dev) if shared else None
+    args = (bf16_dev(x, dev), torch.from_numpy(w).to(dev), torch.from_numpy(ids).to(dev))
+    outs = {}
+    for rows in (E, 200, 1000):
+        bm = _block(fmt, M, k, rows, H, I)
+        blocks = int(np.sum(-(-counts // bm))) + (-(-M // bm) if shared else 0)
+        assert max(blocks * ib, blocks * -(-H // 256)) > cus  # gate_up, down
+        outs[bm] = ops.experts_prefill(*args, _bank_rows(dbank, rows), dsh)
+    # (MXFP4 with a K of 1 mod 4 blocks has no tile of 256)
+    assert set(outs) == ({64, 128} if fmt == "mxfp4" and (hb % 4 == 1 or ib % 4 == 1) else {64, 128, 256})
+    y = outs[64]
+    for other in outs.values():
+        assert torch.equal(y, other)
+    s = rng.choice(M, size=24, replace=False)
+    y_ref = oracle.experts.moe_layer("prefill", x[s], w[s], ids[s] % distinct, bank, sh)
+    got = to_np(y)[s].astype(np.float64)
+    assert np.linalg.norm(got - y_ref) <= 1e-2 * np.linalg.norm(y_ref)
+    assert cosine(got, y_ref) >= COS_TOL, cosine(got, y_ref)
+
+
+@pytest.mark.parametrize("fmt", ["fp8", "mxfp4", "bf16"])
+def test_prefill_bank_rows_up_to_the_limit(dev, fmt):
+    """Banks of 511, 512 and 1023 rows, whose per-expert list fills the LDS beside
+    the largest tiles: the same routes over fewer rows, in another tile, give the
+    same bits."""
+    H, I, k = 256, 384, 8
+    rng = np.random.default_rng(7)
+    bank = to_device_bank(synth.make_bank(fmt, 7, H, I, rng), dev)
+    r = 330 if fmt == "bf16" else 130
+    for rows in (511, 512, 1023):
+        M = r * rows // k + 1
+        g = torch.Generator(device=dev).manual_seed(rows)
+        x = torch.randn((M, H), generator=g, device=dev).to(torch.bfloat16)
+        w, ids = ops.route_softmax_topk(torch.randn((M, 16), generator=g, device=dev), k, True)
+        ids += rows - 16  # the last rows of the bank: nothing lands on the others
+        y = ops.experts_prefill(x, w, ids, _bank_rows(bank, rows))
+        # the same experts as rows 0 to 15 of a bank that puts the weights in the same places
+        few = _bank_rows(bank, rows)
+        few = ops.ExpertBank(few.fmt, *(t[rows - 16:].contiguous() if t is not None else None
+                                        for t in (few.gate_up, few.down, few.gate_up_scale, few.down_scale)))
+        h = 200  # so few tokens a call that it takes 64 or 128 routes per tile
+        assert _block(fmt, h, k, 16, H, I) < 256
+        part = ops.experts_prefill(x[:h].contiguous(), w[:h].contiguous(), (ids[:h] - (rows - 16)).contiguous(), few)
+        assert torch.equal(y[:h], part), rows
+
+
+@pytest.mark.parametrize("offset", [1, 2, 4])
+@pytest.mark.parametrize("M", [1, 33])
+def test_bf16_operands_at_any_element(dev, M, offset):
+    """bf16 tokens and weights that start at any element of their allocation (2,
+    4 and 8 bytes past a 16-byte line): the same bits as aligned ones."""
+    E, H, I, k = 8, 512, 256, 2
+    g = torch.Generator(device=dev).manual_seed(M)
+
+    def at(t):
+        buf = torch.zeros(t.numel() + offset, dtype=t.dtype, device=dev)
+        buf[offset:] = t.reshape(-1)
+        return buf[offset:].view(t.shape)
+
+    gu = (torch.randn((E, 2 * I, H), generator=g, device=dev) * 0.05).to(torch.bfloat16)
+    dn = (torch.randn((E, H, I), generator=g, device=dev) * 0.05).to(torch.bfloat16)
+    x = torch.randn((M, H), generator=g, device=dev).to(torch.bfloat16)
+    w, ids = ops.route_softmax_topk(torch.randn((M, E), generator=g, device=dev), k, True)
+    for fn in (ops.experts_decode, ops.experts_prefill):
+        y = fn(x, w, ids, ops.ExpertBank("bf16", gu, dn))
+        assert torch.equal(y, fn(at(x), w, ids, ops.ExpertBank("bf16", at(gu), at(dn))))
 
 
 def test_prefill_bf16_beyond_2gib(dev):
