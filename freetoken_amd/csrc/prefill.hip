@@ -732,18 +732,28 @@ __global__ void __launch_bounds__(kQThreads) prefill_qgemm_kernel(PrefillGemmArg
     i32x8 wf[4];
     int wcode[4];
     float sw[4];
+    // Row tile j reads weight row 64rg + 16j + r16.  The chunk swizzles depend on
+    // the row's low 3 bits (those of r16) only, so every tile's reads are one
+    // per-lane base of the step plus a compile-time offset.  (A base per tile took
+    // seven more registers than the 256-route MXFP4 kernels have: they spilled,
+    // and read one activation tile at a time.  With these and the scheduling
+    // barrier below: H 4096, I 1536, 64 experts, 3000 tokens 588 -> 558 us; H 7168,
+    // I 2048, 256 experts, 8192 tokens 3166 -> 3008.)
+    const int w0 = 64 * rg + r16;
+    const uint8_t* const w_lo = FMT == FMT_MXFP4 ? st + w0 * 64 + (g ^ swz64(r16)) * 16
+                                                 : st + w0 * 128 + ((2 * g) ^ swz_pair(r16)) * 16;
+    const uint8_t* const w_hi = st + w0 * 128 + ((2 * g + 1) ^ swz_pair(r16)) * 16;  // (not MXFP4)
+    const uint8_t* const w_sc = FMT == FMT_FP8 ? sg + rg * 64 + sq * 4 : sg + w0 * 16 + sq * 4 + g;
     auto read_w = [&](int j) {
-      const int R = 64 * rg + 16 * j + r16;
       if constexpr (FMT != FMT_MXFP4) {
-        const uint8_t* p = st + R * 128;
-        const u32x4 lo = *reinterpret_cast<const u32x4*>(p + (((2 * g) ^ swz_pair(R)) * 16));
-        const u32x4 hi = *reinterpret_cast<const u32x4*>(p + (((2 * g + 1) ^ swz_pair(R)) * 16));
+        const u32x4 lo = *reinterpret_cast<const u32x4*>(w_lo + 2048 * j);
+        const u32x4 hi = *reinterpret_cast<const u32x4*>(w_hi + 2048 * j);
         wf[j] = i32x8{(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)hi[0], (int)hi[1], (int)hi[2], (int)hi[3]};
-        if constexpr (FMT == FMT_FP8) sw[j] = *reinterpret_cast<const float*>(sg + rg * 64 + j * 16 + sq * 4);
+        if constexpr (FMT == FMT_FP8) sw[j] = *reinterpret_cast<const float*>(w_sc + 16 * j);
       } else {
-        const u32x4 v4 = *reinterpret_cast<const u32x4*>(st + R * 64 + ((g ^ swz64(R)) * 16));
+        const u32x4 v4 = *reinterpret_cast<const u32x4*>(w_lo + 1024 * j);
         wf[j] = i32x8{(int)v4[0], (int)v4[1], (int)v4[2], (int)v4[3], 0, 0, 0, 0};
-        wcode[j] = sg[R * 16 + sq * 4 + g];
+        wcode[j] = w_sc[256 * j];
       }
     };
     // Column tile i reads route column (BM/2)ch + 16i + r16.  The chunk swizzle
@@ -808,6 +818,11 @@ __global__ void __launch_bounds__(kQThreads) prefill_qgemm_kernel(PrefillGemmArg
           if (q < kPieces) issue_piece(q, ikb, istg);
       }
       if (i + 1 < NCT) read_x(i + 1, xf[(i + 1) & 1], xs[(i + 1) & 1]);
+      // (held here in the 256-route MXFP4 kernels: short of registers, the
+      // compiler moved these reads behind the MFMAs, which then waited for each
+      // pair of them.  Tile 0 is left to it: the barrier would add tile 1's reads
+      // to the wait of the step's first MFMA)
+      if (FMT == FMT_MXFP4 && BM == 256 && i > 0) __builtin_amdgcn_sched_barrier(0);
       if constexpr (FMT == FMT_BF16) {
         // two K = 32 MFMAs per tile pair, the dependent one four MFMAs later
         const auto half = [](const i32x8& r, int h) {
