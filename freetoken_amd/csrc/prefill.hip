@@ -434,21 +434,24 @@ __device__ __forceinline__ int xcd_major(int b, int n) {
   return x * per + min(x, rem) + i;
 }
 
+struct MNTile {
+  int m, ntile;
+};
+
 // (M block, N tile) of position `local` in a group of nb M blocks x ntiles:
 // chunks of kQChunk M blocks, each chunk sweeping all N tiles.
+// (Returned by value, and from one call per mapping: results written through
+// references from two calls lived in scratch memory, whose loads wait for the
+// copies in flight.)
 template <int kQChunk>
-__device__ __forceinline__ void chunked(int local, int nb, int ntiles, int& m, int& ntile) {
+__device__ __forceinline__ MNTile chunked(int local, int nb, int ntiles) {
   const int full = nb / kQChunk, rem = nb - full * kQChunk;
   const int span = kQChunk * ntiles;
-  if (local < full * span) {
-    const int c = local / span, w = local - c * span;
-    ntile = w / kQChunk;
-    m = c * kQChunk + (w - ntile * kQChunk);
-  } else {
-    const int w = local - full * span;
-    ntile = w / rem;
-    m = full * kQChunk + (w - ntile * rem);
-  }
+  const bool whole = local < full * span;
+  const int c = whole ? local / span : full;
+  const int w = local - c * span, in = whole ? kQChunk : rem;
+  const int ntile = w / in;
+  return {c * kQChunk + (w - ntile * in), ntile};
 }
 
 // Lane index as an asm result: the compiler can neither hoist nor merge it,
@@ -481,8 +484,10 @@ __device__ __forceinline__ bool map_tile_q(const PrefillGemmArgs& a, const int* 
   const int total = routed + a.shared_blocks * a.ntiles;
   if (b >= total) return false;
   const int wg = xcd_major(b, total);
-  if (wg < routed) {
-    int owner = -1;  // largest e whose first tile is <= wg
+  int local = wg - routed, nb = a.shared_blocks, b0 = 0, owner = 0;
+  const bool shared = wg >= routed;
+  if (!shared) {
+    owner = -1;  // largest e whose first tile is <= wg
     for (int e0 = 0; e0 < E; e0 += 4 * kWave) {
       int first[4];  // four reads in flight (entries past the last expert: its neighbours)
       const int l = fresh_lane();
@@ -492,18 +497,15 @@ __device__ __forceinline__ bool map_tile_q(const PrefillGemmArgs& a, const int* 
       for (int u = 0; u < 4; ++u) owner += __popcll(__ballot(e0 + u * kWave + l < E && first[u] * a.ntiles <= wg));
     }
     owner = __builtin_amdgcn_readfirstlane(owner);
-    const int b0 = __builtin_amdgcn_readfirstlane(s_blk[owner]);
-    const int nb = __builtin_amdgcn_readfirstlane(s_blk[owner + 1]) - b0;
-    int m;
-    chunked<kQChunk>(wg - b0 * a.ntiles, nb, a.ntiles, m, t.ntile);
-    t.shared = false;
-    t.expert = owner;
-    t.mblock = b0 + m;
-    return true;
+    b0 = __builtin_amdgcn_readfirstlane(s_blk[owner]);
+    nb = __builtin_amdgcn_readfirstlane(s_blk[owner + 1]) - b0;
+    local = wg - b0 * a.ntiles;
   }
-  chunked<kQChunk>(wg - routed, a.shared_blocks, a.ntiles, t.mblock, t.ntile);
-  t.shared = true;
-  t.expert = 0;
+  const MNTile mn = chunked<kQChunk>(local, nb, a.ntiles);
+  t.shared = shared;
+  t.expert = owner;
+  t.mblock = b0 + mn.m;
+  t.ntile = mn.ntile;
   return true;
 }
 

@@ -62,6 +62,18 @@ def test_validation_errors_without_launch():
     assert rc == _lib.FTMOE_ERR_UNSUPPORTED
 
 
+def test_prefill_gemms_use_no_scratch_memory():
+    """A load from scratch memory waits for every copy in flight, so the
+    persistent prefill GEMMs keep nothing there: the private segment of each of
+    them, in the library's kernel metadata, is empty."""
+    blob = _lib.LIB_PATH.read_bytes()
+    key = rb"\.private_segment_fixed_size"
+    found = re.findall(rb"\.name(?:\xd9.|[\xa0-\xbf])(_ZN5ftmoe20prefill_qgemm_kernel\w+E)\xbb" + key + rb"(.)",
+                       blob, re.DOTALL)
+    assert len(found) >= 18  # three formats, two GEMMs, three tiles
+    assert {name: size for name, size in found if size != b"\x00"} == {}
+
+
 def test_align_sizes_formula():
     from freetoken_amd.ops import align_sizes
 
