@@ -478,29 +478,45 @@ struct QTile {
 // total.  The owner of a position is found by the whole wave at once (one
 // ballot per 64 experts): a binary search over the regions in global memory
 // was a chain of dependent loads at every tile, each of whose waits drained
-// the copies in flight.
-template <int kQChunk>
+// the copies in flight.  A workgroup's first tile, with nothing in flight yet,
+// takes that search in scalar registers instead of waiting for s_blk (small
+// calls, whose workgroups have one tile: H 1280, I 640, 16 experts, 2048 tokens,
+// gate_up 30.6 -> 29.9 us).
+template <int kQChunk, int BM, bool kFirst>
 __device__ __forceinline__ bool map_tile_q(const PrefillGemmArgs& a, const int* s_blk, int b, QTile& t) {
   const int E = a.num_experts;
-  const int routed = __builtin_amdgcn_readfirstlane(s_blk[E]) * a.ntiles;
+  auto first_block = [&](int e) -> int {
+    if constexpr (kFirst) return a.cum[e] / BM;
+    else return __builtin_amdgcn_readfirstlane(s_blk[e]);
+  };
+  const int routed = first_block(E) * a.ntiles;
   const int total = routed + a.shared_blocks * a.ntiles;
   if (b >= total) return false;
   const int wg = xcd_major(b, total);
   int local = wg - routed, nb = a.shared_blocks, b0 = 0, owner = 0;
   const bool shared = wg >= routed;
-  if (!shared) {
-    owner = -1;  // largest e whose first tile is <= wg
-    for (int e0 = 0; e0 < E; e0 += 4 * kWave) {
-      int first[4];  // four reads in flight (entries past the last expert: its neighbours)
-      const int l = fresh_lane();
+  if (!shared) {  // owner: the largest e whose first tile is <= wg
+    if constexpr (kFirst) {
+      int hi = E;
+      while (hi - owner > 1) {
+        const int mid = (owner + hi) >> 1;
+        if (first_block(mid) * a.ntiles <= wg) owner = mid;
+        else hi = mid;
+      }
+    } else {
+      owner = -1;
+      for (int e0 = 0; e0 < E; e0 += 4 * kWave) {
+        int first[4];  // four reads in flight (entries past the last expert: its neighbours)
+        const int l = fresh_lane();
 #pragma unroll
-      for (int u = 0; u < 4; ++u) first[u] = s_blk[min(e0 + u * kWave + l, E)];
+        for (int u = 0; u < 4; ++u) first[u] = s_blk[min(e0 + u * kWave + l, E)];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) owner += __popcll(__ballot(e0 + u * kWave + l < E && first[u] * a.ntiles <= wg));
+        for (int u = 0; u < 4; ++u) owner += __popcll(__ballot(e0 + u * kWave + l < E && first[u] * a.ntiles <= wg));
+      }
+      owner = __builtin_amdgcn_readfirstlane(owner);
     }
-    owner = __builtin_amdgcn_readfirstlane(owner);
-    b0 = __builtin_amdgcn_readfirstlane(s_blk[owner]);
-    nb = __builtin_amdgcn_readfirstlane(s_blk[owner + 1]) - b0;
+    b0 = first_block(owner);
+    nb = first_block(owner + 1) - b0;
     local = wg - b0 * a.ntiles;
   }
   const MNTile mn = chunked<kQChunk>(local, nb, a.ntiles);
@@ -579,12 +595,11 @@ __global__ void __launch_bounds__(kQThreads) prefill_qgemm_kernel(PrefillGemmArg
   const uint32_t rb = FMT == FMT_BF16 ? 2u * K : FMT == FMT_FP8 ? 1u * K : static_cast<uint32_t>(K) / 2;
   const uint32_t xb = FMT == FMT_BF16 ? 2u * K : 1u * K;
 
-  for (int e = tid; e <= a.num_experts; e += kQThreads) s_blk[e] = a.cum[e] / BM;
-  __syncthreads();
+  for (int e = tid; e <= a.num_experts; e += kQThreads) s_blk[e] = a.cum[e] / BM;  // (published with the first routes)
   int v = blockIdx.x;
   QTile cur;
   constexpr int kChunk = q_chunk<FMT, GATE_UP, BM>();
-  if (!map_tile_q<kChunk>(a, s_blk, v, cur)) return;
+  if (!map_tile_q<kChunk, BM, true>(a, s_blk, v, cur)) return;
 
   auto n0_of = [&](const QTile& t) -> int { return GATE_UP ? t.ntile * (kQRows / 2) : t.ntile * kQRows; };
   // first weight row of tile j of row group q, relative to the tile's first row n0
@@ -1069,7 +1084,7 @@ __global__ void __launch_bounds__(kQThreads) prefill_qgemm_kernel(PrefillGemmArg
         if (d < nkb) issue(d, (g0 + d) % S, gb);
     }
     QTile nxt;
-    const bool has_next = map_tile_q<kChunk>(a, s_blk, v + static_cast<int>(gridDim.x), nxt);
+    const bool has_next = map_tile_q<kChunk, BM, false>(a, s_blk, v + static_cast<int>(gridDim.x), nxt);
     // the next tile's first steps ride in this tile's last D steps, unless its
     // first scale group's buffer would still be in use (kGroups 2 and a last
     // group shorter than D)
