@@ -568,7 +568,7 @@ __device__ __forceinline__ void pin(f32x4& v) { asm volatile("" : "+v"(v)); }
 
 __device__ __forceinline__ uint64_t uniform_u64(uint64_t v) { return readlane_u64(v, 0); }
 
-template <int FMT, int GATE_UP, int BM>
+template <int FMT, int GATE_UP, int BM, bool NT>
 __global__ void __launch_bounds__(kQThreads) prefill_qgemm_kernel(PrefillGemmArgs a) {
   using L = QLds<FMT, BM>;
   constexpr int S = L::kStages;
@@ -1039,8 +1039,7 @@ __global__ void __launch_bounds__(kQThreads) prefill_qgemm_kernel(PrefillGemmArg
           const int route = s_route[b][(BM / 2) * ch + 16 * (p * CT + (c >> 4)) + (c & 15)];
           if (route < lim_col && rows_in) {
             u32x4* const dst = reinterpret_cast<u32x4*>(base + static_cast<size_t>(route) * a.N + nrow0 + 8 * chunk);
-            // (256-route tiles mean outputs far beyond L2: 8192 tokens, H 7168: down and combine 1% faster)
-            if constexpr (BM == 256) __builtin_nontemporal_store(v, dst);
+            if constexpr (NT) __builtin_nontemporal_store(v, dst);
             else *dst = v;
           }
         }
@@ -1198,14 +1197,14 @@ static int q_cu_count() {
   return cached;
 }
 
-template <int FMT, int GU, int BM>
+template <int FMT, int GU, int BM, bool NT = false>
 static hipError_t launch_qgemm_t(PrefillGemmArgs a, hipStream_t stream) {
   // the ring, the scale groups, then one int per expert (and the total)
   const int lds = QLds<FMT, BM>::kFixed + (a.num_experts + 1) * 4;
   static bool attr = false;
   if (!attr) {
     const hipError_t err =
-        hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_qgemm_kernel<FMT, GU, BM>),
+        hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_qgemm_kernel<FMT, GU, BM, NT>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 4096);
     if (err != hipSuccess) return err;
     attr = true;
@@ -1217,15 +1216,27 @@ static hipError_t launch_qgemm_t(PrefillGemmArgs a, hipStream_t stream) {
   const long long tiles = static_cast<long long>(a.max_blocks + a.shared_blocks) * a.ntiles;
   const int wgs = static_cast<int>(std::min<long long>(tiles, q_cu_count()));
   if (wgs <= 0) return hipSuccess;
-  hipLaunchKernelGGL((prefill_qgemm_kernel<FMT, GU, BM>), dim3(wgs), dim3(kQThreads), lds, stream, a);
+  hipLaunchKernelGGL((prefill_qgemm_kernel<FMT, GU, BM, NT>), dim3(wgs), dim3(kQThreads), lds, stream, a);
   return hipGetLastError();
 }
+
+// Down outputs above this are stored nontemporally: they pass the 256 MB
+// memory-side cache before the combine reads them.  Measured (us of the call,
+// plain / nontemporal): FP8 145 MB 338 / 344, 303 MB 514.7 / 519.7, 397 MB 1098 /
+// 1106, 470 MB 1825 / 1819, 1.06 GB 3862 / 3834; MXFP4 1.06 GB 3097 / 3059.  A
+// test of the size inside the kernel cost the largest call 1%, so the choice is
+// a variant's.
+constexpr size_t kStreamedOutputs = size_t{448} << 20;
 
 template <int FMT, int GU>
 static hipError_t launch_qgemm_bm(const PrefillGemmArgs& a, hipStream_t stream) {
   if (a.block == 64) return launch_qgemm_t<FMT, GU, 64>(a, stream);
   if (a.block == 128) return launch_qgemm_t<FMT, GU, 128>(a, stream);
-  if (a.block == 256) return launch_qgemm_t<FMT, GU, 256>(a, stream);
+  if (a.block == 256) {
+    const size_t out_bytes = (static_cast<size_t>(a.numel) + (a.shared_blocks ? a.M : 0)) * a.N * 2;
+    if (!GU && out_bytes > kStreamedOutputs) return launch_qgemm_t<FMT, GU, 256, !GU>(a, stream);
+    return launch_qgemm_t<FMT, GU, 256>(a, stream);
+  }
   return hipErrorInvalidValue;
 }
 
