@@ -170,10 +170,11 @@ PrefillLayout prefill_layout(void* ws, int M, int k, const ftmoe_bank* bank, con
   const int H = bank->hidden, I = bank->inter;
   ftmoe_align_sizes(numel, bank->num_rows, ftmoe::prefill_block_size(bank->format, M, k, bank->num_rows, H, I),
                     &L.max_padded, &L.max_blocks);
-  // a workspace of the largest M serves the smaller ones: the bf16 calls past
-  // 2 GiB go back from 256 routes per block to 128, and keep the room of 256
+  // a workspace of the largest M serves the smaller ones: the few calls that go
+  // back from 256 routes per block to 128 (bf16 past 2 GiB, MXFP4 past 2^16
+  // blocks) keep the room of 256
   int room = L.max_padded, unused = 0;
-  if (!ftmoe::prefill_operands_fit(bank->format, M, k, H, I))
+  if (static_cast<int64_t>(numel) > 320ll * bank->num_rows)
     ftmoe_align_sizes(numel, bank->num_rows, 256, &room, &unused);
   L.sorted = c.take<int32_t>(std::max(room, L.max_padded));
   L.expert_ids = c.take<int32_t>(L.max_blocks);

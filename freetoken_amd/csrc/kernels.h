@@ -1,6 +1,8 @@
 // Argument structs and launch entry points shared by the kernels and the C ABI.
 #pragma once
 
+#include <algorithm>
+
 #include "ftmoe_common.h"
 
 namespace ftmoe {
@@ -175,16 +177,21 @@ inline bool prefill_operands_fit(int fmt, int M, int k, int H, int I) {
 // / 3303), but at r = 137 an even one is already 8% slower at 128.
 // bf16 of the first shape: r = 38 267 / 271 / 311, r = 87 355 / 302 / 338, r =
 // 256 628 / 487 / 507 (uneven 647 / 515 / 564), r = 512 1115 / 825 / 803.
-// The MXFP4 tiles of 256 hold two groups of scales, which costs their copies'
-// overlap across tiles when K / 128 leaves a remainder of 1 by four, and up to
-// 511 experts in LDS: 128 takes those calls.
+// Beyond those, 128 where its tiles of both GEMMs fit one round of the 256 CUs:
+// those of 256 then leave half of them idle.  Blocks of 128 / 256, H 1280, I 640,
+// 16 experts, top-4: 240 tiles of 128 (1300 tokens) FP8 56.0 / 67.7, MXFP4 53.4 /
+// 65.7, bf16 57.6 / 71.4; 290 (1600 tokens) MXFP4 72.4 / 66.4.
+// (MXFP4 tiles of 256 count M blocks in 16 bits, for up to 1023 rows in LDS: 600
+// experts, H 2048, I 512, 11250 tokens, blocks of 128 774, 256 666.)
 inline int prefill_block_size(int fmt, int M, int k, int rows, int H, int I) {
   // (the register-staged bf16 GEMM tiles 128)
   if (fmt == FMT_BF16 && !prefill_operands_fit(fmt, M, k, H, I)) return 128;
   const long long routes = static_cast<long long>(M) * k;
   if (routes <= 48ll * rows) return 64;
   if (routes <= (fmt == FMT_BF16 ? 320ll : 120ll) * rows) return 128;
-  if (fmt == FMT_MXFP4 && (rows > 511 || H / 128 % 4 == 1 || I / 128 % 4 == 1)) return 128;
+  // (the mean last block of a row is half full)
+  if ((routes / 128 + rows / 2) * std::max(I / 128, (H + 255) / 256) <= 256) return 128;
+  if (fmt == FMT_MXFP4 && routes > 256ll * (UINT16_MAX - kPrefillMaxRows)) return 128;
   return 256;
 }
 

@@ -382,6 +382,7 @@ __global__ void __launch_bounds__(kPThreads) prefill_gemm_kernel(PrefillGemmArgs
 constexpr int kQRows = 256;   // weight rows per workgroup
 constexpr int kQThreads = 512;
 constexpr int kXcds = 8;
+constexpr int kQDynamicLds = 160 * 1024 - 4096;  // beside the tiles' route and weight lists
 // M blocks per chunk of the schedule (see map_tile_q): [FP8, MXFP4][gate_up, down].
 // Measured on C5 (interleaved A/B, ms): FP8 gate_up 4 -> 2.23-2.24, 8 -> 2.19-2.20,
 // 16 -> 2.22, 2 -> 2.32; FP8 down 4 -> 1.25-1.26, 2 -> 1.20, 1 -> 1.22; MXFP4
@@ -426,8 +427,11 @@ struct QLds {
   static constexpr int kXS = FMT == FMT_FP8 ? BM * 16 : FMT == FMT_MXFP4 ? BM * 4 : 0;
   static constexpr int kGroup = kWS + kXS;
   static constexpr int kGroups = BM == 256 ? 2 : 3;
-  // LDS before the expert list
+  // LDS before the expert list, whose entries are halved where 1024 of them
+  // would not fit (prefill_block_size keeps such calls below 2^16 blocks)
   static constexpr int kFixed = kRing + kGroups * kGroup;
+  using Blk = std::conditional_t<FMT == FMT_MXFP4 && BM == 256, uint16_t, int>;
+  static_assert(kFixed + (kPrefillMaxRows + 1) * sizeof(Blk) <= kQDynamicLds, "the expert list fits beside the ring");
 };
 
 __device__ __forceinline__ int xcd_major(int b, int n) {
@@ -482,12 +486,12 @@ struct QTile {
 // takes that search in scalar registers instead of waiting for s_blk (small
 // calls, whose workgroups have one tile: H 1280, I 640, 16 experts, 2048 tokens,
 // gate_up 30.6 -> 29.9 us).
-template <int kQChunk, int BM, bool kFirst>
-__device__ __forceinline__ bool map_tile_q(const PrefillGemmArgs& a, const int* s_blk, int b, QTile& t) {
+template <int kQChunk, int BM, bool kFirst, typename Blk>
+__device__ __forceinline__ bool map_tile_q(const PrefillGemmArgs& a, const Blk* s_blk, int b, QTile& t) {
   const int E = a.num_experts;
   auto first_block = [&](int e) -> int {
     if constexpr (kFirst) return a.cum[e] / BM;
-    else return __builtin_amdgcn_readfirstlane(s_blk[e]);
+    else return __builtin_amdgcn_readfirstlane(static_cast<int>(s_blk[e]));
   };
   const int routed = first_block(E) * a.ntiles;
   const int total = routed + a.shared_blocks * a.ntiles;
@@ -577,7 +581,7 @@ __global__ void __launch_bounds__(kQThreads) prefill_qgemm_kernel(PrefillGemmArg
   constexpr bool kQuant = L::kQuant;
   // ring of stages, scale groups, then the first M block of every expert ([num_experts + 1])
   extern __shared__ __attribute__((aligned(16))) uint8_t q_lds[];
-  int* const s_blk = reinterpret_cast<int*>(q_lds + L::kFixed);
+  typename L::Blk* const s_blk = reinterpret_cast<typename L::Blk*>(q_lds + L::kFixed);
   // per tile parity: each route column's route (shared tiles: token); padding
   // columns hold a value at or past the tile's limit (col_limit)
   __shared__ int s_route[2][BM];
@@ -595,7 +599,7 @@ __global__ void __launch_bounds__(kQThreads) prefill_qgemm_kernel(PrefillGemmArg
   const uint32_t rb = FMT == FMT_BF16 ? 2u * K : FMT == FMT_FP8 ? 1u * K : static_cast<uint32_t>(K) / 2;
   const uint32_t xb = FMT == FMT_BF16 ? 2u * K : 1u * K;
 
-  for (int e = tid; e <= a.num_experts; e += kQThreads) s_blk[e] = a.cum[e] / BM;  // (published with the first routes)
+  for (int e = tid; e <= a.num_experts; e += kQThreads) s_blk[e] = static_cast<typename L::Blk>(a.cum[e] / BM);  // (published with the first routes)
   int v = blockIdx.x;
   QTile cur;
   constexpr int kChunk = q_chunk<FMT, GATE_UP, BM>();
@@ -1200,12 +1204,12 @@ static int q_cu_count() {
 template <int FMT, int GU, int BM, bool NT = false>
 static hipError_t launch_qgemm_t(PrefillGemmArgs a, hipStream_t stream) {
   // the ring, the scale groups, then one int per expert (and the total)
-  const int lds = QLds<FMT, BM>::kFixed + (a.num_experts + 1) * 4;
+  const int lds = QLds<FMT, BM>::kFixed + (a.num_experts + 1) * static_cast<int>(sizeof(typename QLds<FMT, BM>::Blk));
   static bool attr = false;
   if (!attr) {
     const hipError_t err =
         hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_qgemm_kernel<FMT, GU, BM, NT>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024 - 4096);
+                            hipFuncAttributeMaxDynamicSharedMemorySize, kQDynamicLds);
     if (err != hipSuccess) return err;
     attr = true;
   }

@@ -142,11 +142,21 @@ def test_prefill_activation_variants(dev, fmt, activation):
     assert max_rel(y_silu, y_ref) > 4 * MAX_REL_TOL
 
 
+def _bank_rows(bank, rows):
+    """The device bank's rows in turn, `rows` of them."""
+    def take(t):
+        idx = torch.arange(rows, device=bank.gate_up.device) % t.shape[0]
+        return t.view(torch.uint8)[idx].view(t.dtype)
+
+    return ops.ExpertBank(bank.fmt, *(take(t) if t is not None else None
+                                      for t in (bank.gate_up, bank.down, bank.gate_up_scale, bank.down_scale)))
+
+
 @pytest.mark.parametrize("H,I", [(640, 384), (128, 1152), (1024, 128)])
 @pytest.mark.parametrize("fmt,block,n,E,E2", [
-    ("fp8", 64, 2, 16, 3), ("fp8", 128, 1, 4, 16), ("fp8", 256, 1, 4, 16),
-    ("mxfp4", 64, 2, 16, 3), ("mxfp4", 128, 1, 4, 16), ("mxfp4", 256, 1, 4, 16),
-    ("bf16", 64, 2, 16, 3), ("bf16", 128, 1, 4, 16), ("bf16", 256, 2, 3, 16),
+    ("fp8", 64, 2, 16, 3), ("fp8", 128, 1, 4, 16), ("fp8", 256, 24, 4, 128),
+    ("mxfp4", 64, 2, 16, 3), ("mxfp4", 128, 1, 4, 16), ("mxfp4", 256, 24, 4, 128),
+    ("bf16", 64, 2, 16, 3), ("bf16", 128, 1, 4, 16), ("bf16", 256, 24, 4, 128),
 ])
 def test_prefill_block_sizes(dev, fmt, block, n, E, E2, H, I):
     """Every routes-per-tile variant of the GEMMs at its edges: one expert with
@@ -159,8 +169,6 @@ def test_prefill_block_sizes(dev, fmt, block, n, E, E2, H, I):
     whose bf16 rounding, and with it its e4m3 code, falls the other way (the
     sums differ in their last bit) moves one output row by up to 1/16 of that
     product, which the maximum over few outputs would show as 2-3%."""
-    if fmt == "mxfp4" and block == 256:  # (those with a K of 1 mod 4 blocks take 128)
-        H, I = {640: (768, 384), 128: (256, 1408), 1024: (1024, 256)}[H]
     rng = np.random.default_rng(block + H)
     flat = np.repeat(np.arange(3, dtype=np.int32), [n * block, n * block + 1, 1])
     ids = rng.permutation(flat).reshape(-1, 2)
@@ -171,21 +179,11 @@ def test_prefill_block_sizes(dev, fmt, block, n, E, E2, H, I):
     x = synth.activations(rng, M, H)
     y_ref = oracle.experts.moe_layer("prefill", x, w, ids, bank, sh)
     y, y2 = (ops.experts_prefill(bf16_dev(x, dev), torch.from_numpy(w).to(dev), torch.from_numpy(ids).to(dev),
-                                 to_device_bank(bank, dev, slice(0, r)), to_device_bank(sh, dev)) for r in (E, E2))
+                                 _bank_rows(to_device_bank(bank, dev), r), to_device_bank(sh, dev)) for r in (E, E2))
     assert torch.equal(y, y2)
     got = to_np(y).astype(np.float64)
     assert np.linalg.norm(got - y_ref) <= 1e-2 * np.linalg.norm(y_ref)
     assert cosine(got, y_ref) >= COS_TOL, cosine(got, y_ref)
-
-
-def _bank_rows(bank, rows):
-    """The device bank's rows in turn, `rows` of them."""
-    def take(t):
-        idx = torch.arange(rows, device=bank.gate_up.device) % t.shape[0]
-        return t.view(torch.uint8)[idx].view(t.dtype)
-
-    return ops.ExpertBank(bank.fmt, *(take(t) if t is not None else None
-                                      for t in (bank.gate_up, bank.down, bank.gate_up_scale, bank.down_scale)))
 
 
 @pytest.mark.parametrize("hb,ib,shared", [(5, 1, True), (6, 2, False), (7, 3, True), (9, 4, False), (1, 6, True),
@@ -215,8 +213,7 @@ def test_prefill_many_tiles_per_workgroup(dev, fmt, hb, ib, shared):
         blocks = int(np.sum(-(-counts // bm))) + (-(-M // bm) if shared else 0)
         assert max(blocks * ib, blocks * -(-H // 256)) > cus  # gate_up, down
         outs[bm] = ops.experts_prefill(*args, _bank_rows(dbank, rows), dsh)
-    # (MXFP4 with a K of 1 mod 4 blocks has no tile of 256)
-    assert set(outs) == ({64, 128} if fmt == "mxfp4" and (hb % 4 == 1 or ib % 4 == 1) else {64, 128, 256})
+    assert set(outs) == {64, 128, 256}
     y = outs[64]
     for other in outs.values():
         assert torch.equal(y, other)
@@ -242,6 +239,7 @@ def test_prefill_bank_rows_up_to_the_limit(dev, fmt):
         x = torch.randn((M, H), generator=g, device=dev).to(torch.bfloat16)
         w, ids = ops.route_softmax_topk(torch.randn((M, 16), generator=g, device=dev), k, True)
         ids += rows - 16  # the last rows of the bank: nothing lands on the others
+        assert _block(fmt, M, k, rows, H, I) == 256
         y = ops.experts_prefill(x, w, ids, _bank_rows(bank, rows))
         # the same experts as rows 0 to 15 of a bank that puts the weights in the same places
         few = _bank_rows(bank, rows)
