@@ -166,8 +166,8 @@ inline bool prefill_operands_fit(int fmt, int M, int k, int H, int I) {
 }
 
 // Routes per M block of the prefill GEMMs (the align block size): 256, or by
-// the mean number of routes per expert r = M k / rows 64 (r <= 48) or 128 (r <=
-// 120; bf16 r <= 320): a tile of 256 is then mostly padding.
+// the mean number of routes per expert r = M k / rows 64 (r <= 24, on small grids
+// r <= 48) or 128 (r <= 120; bf16 r <= 320): a tile of 256 is then mostly padding.
 // Measured (us, blocks of 64 / 128 / 256): FP8 H 2048, I 768, 128 experts,
 // top-8, r = 31 165 / 172 / 206, r = 69 214 / 189 / 223, r = 112 252 / 223 /
 // 239, r = 137 287 / 263 / 243; MXFP4 of that shape r = 31 118 / 130 / 179, r =
@@ -177,6 +177,14 @@ inline bool prefill_operands_fit(int fmt, int M, int k, int H, int I) {
 // / 3303), but at r = 137 an even one is already 8% slower at 128.
 // bf16 of the first shape: r = 38 267 / 271 / 311, r = 87 355 / 302 / 338, r =
 // 256 628 / 487 / 507 (uneven 647 / 515 / 564), r = 512 1115 / 825 / 803.
+// The lower line: on a grid of many rounds, where an uneven routing puts most
+// routes on few experts, 64 pays for its halved reuse of every weight read (Zipf
+// 1.1, blocks of 64 / 128 / 256: FP8 H 2688, I 1664, 248 experts, top-6, r = 30
+// 266 / 243 / 257, r = 47 348 / 287 / 304; H 7168, I 2048, 128 experts, r = 47
+// 611 / 521 / 540; even ones 1004 / 999 / 1331 and 1076 / 1000 / 1338, MXFP4 662
+// / 686 / 1056 and 750 / 766 / 1106); up to 1024 tiles of gate_up (one block per
+// expert) it stays ahead (r = 47, grouped top-8 of the first shape, uneven, FP8
+// 106 / 103 / 131, MXFP4 91 / 92 / 94; 64 experts, H 4096, I 1024 223 / 238 / 315).
 // Beyond those, 128 where its tiles of both GEMMs fit one round of the 256 CUs:
 // those of 256 then leave half of them idle.  Blocks of 128 / 256, H 1280, I 640,
 // 16 experts, top-4: 240 tiles of 128 (1300 tokens) FP8 56.0 / 67.7, MXFP4 53.4 /
@@ -187,7 +195,7 @@ inline int prefill_block_size(int fmt, int M, int k, int rows, int H, int I) {
   // (the register-staged bf16 GEMM tiles 128)
   if (fmt == FMT_BF16 && !prefill_operands_fit(fmt, M, k, H, I)) return 128;
   const long long routes = static_cast<long long>(M) * k;
-  if (routes <= 48ll * rows) return 64;
+  if (routes <= 24ll * rows || (routes <= 48ll * rows && rows * (I / 128) <= 1024)) return 64;
   if (routes <= (fmt == FMT_BF16 ? 320ll : 120ll) * rows) return 128;
   // (the mean last block of a row is half full)
   if ((routes / 128 + rows / 2) * std::max(I / 128, (H + 255) / 256) <= 256) return 128;
