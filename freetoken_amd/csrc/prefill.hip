@@ -566,6 +566,14 @@ template <int FMT>
 __device__ __forceinline__ int swz_b(int line) { return FMT == FMT_MXFP4 ? (line & 7) : swz_pair(line); }
 __device__ __forceinline__ int swz64(int line) { return (line >> 1) & 3; }
 
+// Position of a running count in a ring of N.  (Unsigned: the signed remainders
+// were a dozen more scalar operations at the head of every step, before its
+// first LDS read: FP8 1-13 tiles a workgroup 0.3-0.8% of the call.)
+template <int N>
+__device__ __forceinline__ int ring(int i) {
+  return static_cast<int>(static_cast<unsigned>(i) % N);
+}
+
 // Empty asm that keeps the value's update at this point of the instruction
 // stream (no code is emitted).
 __device__ __forceinline__ void pin(f32x4& v) { asm volatile("" : "+v"(v)); }
@@ -731,7 +739,7 @@ __global__ void __launch_bounds__(kQThreads) prefill_qgemm_kernel(PrefillGemmArg
     }
   };
   auto issue = [&](int kb, int stg, int gb) {
-    if ((kb & 3) == 0) issue_scales(kb, (gb + (kb >> 2)) % L::kGroups);
+    if ((kb & 3) == 0) issue_scales(kb, ring<L::kGroups>(gb + (kb >> 2)));
 #pragma unroll
     for (int q = 0; q < kPieces; ++q) issue_piece(q, kb, stg);
   };
@@ -749,8 +757,8 @@ __global__ void __launch_bounds__(kQThreads) prefill_qgemm_kernel(PrefillGemmArg
   constexpr int kPer = NCT == 8 ? 2 : (kPieces + NCT - 1) / NCT;  // pieces per column tile
   auto compute = [&](int kb, int stg, int gb, int ikb, int istg, int igb) {
     const uint8_t* st = q_lds + stg * L::kStage;
-    if (ikb >= 0 && (ikb & 3) == 0) issue_scales(ikb, (igb + (ikb >> 2)) % L::kGroups);
-    const uint8_t* sg = scale_group((gb + (kb >> 2)) % L::kGroups);
+    if (ikb >= 0 && (ikb & 3) == 0) issue_scales(ikb, ring<L::kGroups>(igb + (ikb >> 2)));
+    const uint8_t* sg = scale_group(ring<L::kGroups>(gb + (kb >> 2)));
     const int sq = kb & 3;  // step of the group
     i32x8 wf[4];
     int wcode[4];
@@ -1084,7 +1092,7 @@ __global__ void __launch_bounds__(kQThreads) prefill_qgemm_kernel(PrefillGemmArg
     if (!ahead) {
 #pragma unroll
       for (int d = 0; d < D; ++d)
-        if (d < nkb) issue(d, (g0 + d) % S, gb);
+        if (d < nkb) issue(d, ring<S>(g0 + d), gb);
     }
     QTile nxt;
     const bool has_next = map_tile_q<kChunk, BM, false>(a, s_blk, v + static_cast<int>(gridDim.x), nxt);
@@ -1115,10 +1123,10 @@ __global__ void __launch_bounds__(kQThreads) prefill_qgemm_kernel(PrefillGemmArg
     int kb = 0;
     for (; kb < nkb - D; ++kb) {
       if constexpr (kSpread) {
-        compute(kb, (g0 + kb) % S, gb, kb + D, (g0 + kb + D) % S, gb);
+        compute(kb, ring<S>(g0 + kb), gb, kb + D, ring<S>(g0 + kb + D), gb);
       } else {
-        issue(kb + D, (g0 + kb + D) % S, gb);
-        compute(kb, (g0 + kb) % S, gb, -1, 0, 0);
+        issue(kb + D, ring<S>(g0 + kb + D), gb);
+        compute(kb, ring<S>(g0 + kb), gb, -1, 0, 0);
       }
       wait_vm<(D - 1) * L::kDmaPerStep>();
       wait_lgkm0();
@@ -1137,10 +1145,10 @@ __global__ void __launch_bounds__(kQThreads) prefill_qgemm_kernel(PrefillGemmArg
     if (cross) setup(nxt, buf ^ 1);
     for (; kb < nkb; ++kb) {
       if constexpr (kSpread) {
-        compute(kb, (g0 + kb) % S, gb, cross ? kb + D - nkb : -1, (g0 + kb + D) % S, gbn);
+        compute(kb, ring<S>(g0 + kb), gb, cross ? kb + D - nkb : -1, ring<S>(g0 + kb + D), gbn);
       } else {
-        if (cross) issue(kb + D - nkb, (g0 + kb + D) % S, gbn);
-        compute(kb, (g0 + kb) % S, gb, -1, 0, 0);
+        if (cross) issue(kb + D - nkb, ring<S>(g0 + kb + D), gbn);
+        compute(kb, ring<S>(g0 + kb), gb, -1, 0, 0);
       }
       if (kb + 1 < nkb) {
         if (cross) wait_vm<(D - 1) * L::kDmaPerStep>();
@@ -1152,13 +1160,13 @@ __global__ void __launch_bounds__(kQThreads) prefill_qgemm_kernel(PrefillGemmArg
     // the stage of this tile's last step: the next tile's first D steps ride
     // in the other stages, and its step D is issued after the barrier that
     // starts its K loop
-    epilogue(cur, buf, q_lds + ((g0 + nkb + D) % S) * L::kStage);
+    epilogue(cur, buf, q_lds + (ring<S>(g0 + nkb + D)) * L::kStage);
     if (!has_next) break;
     ahead = cross;
     cur = nxt;
     buf ^= 1;
     g0 += nkb;
-    gb = gbn % L::kGroups;
+    gb = ring<L::kGroups>(gbn);
     v += static_cast<int>(gridDim.x);
     if (!ahead) setup(cur, buf);
   }
