@@ -731,7 +731,8 @@ int ftmoe_experts_prefill(const void* x, int M, int top_k, const float* topk_w, 
   const uint16_t* xb = static_cast<const uint16_t*>(x);
   const int qmode = fmt == FTMOE_FMT_MXFP4 ? 1 : 0;
   if (fmt != FTMOE_FMT_BF16) {
-    rc = check_hip(ftmoe::launch_act_quant(qmode, xb, M, H, ftmoe::act_scale_stride(H), L.xq, L.xs, stream), "experts_prefill x quant");
+    rc = check_hip(ftmoe::launch_act_quant(qmode, xb, M, H, ftmoe::act_scale_stride(H), L.xq, L.xs, stream),
+                   "experts_prefill x quant");
     if (rc) return rc;
   }
   g_timer.mark();

@@ -88,16 +88,16 @@ struct RawA<FMT_MXFP4> {
 // Weights and activations are read through buffer descriptors (make_rsrc,
 // buf_x4): base in SGPRs, 32-bit lane offsets, the K-block offset in soffset.
 
+// The register path (load_raw to gemv_tile): MXFP4 with K not a multiple of 256;
+// everything else takes the LDS path (gemv_tile_dma).
 // Weight bytes of one lane for K block kb: the lane's row starts at voff
 // (row * row_bytes + a_group_bytes * lane group); the K block adds kb * 128
-// values.  MXFP4: the lane's e8m0 code sits at coff + kb * 4 of the
-// code rows (sr).  `dead` is 0 or kOutOfRange: a dead K block (past the wave's
-// range) is still issued, so every K step issues the same loads and the
-// wait counts stay exact, but it reads zeros without touching memory.
-template <int FMT>
+// values.  The lane's e8m0 code sits at coff + kb * 4 of the code rows (sr).
+// `dead` is 0 or kOutOfRange: a dead K block (past the wave's range) is still
+// issued, so every K step issues the same loads and the wait counts stay exact,
+// but it reads zeros without touching memory.
 __device__ __forceinline__ void load_raw(__amdgpu_buffer_rsrc_t wr, __amdgpu_buffer_rsrc_t sr, uint32_t voff,
-                                         uint32_t coff, int kb, uint32_t dead, RawA<FMT>& r) {
-  static_assert(FMT == FMT_MXFP4, "the other formats take the LDS path (gemv_tile_dma)");
+                                         uint32_t coff, int kb, uint32_t dead, RawA<FMT_MXFP4>& r) {
   r.v[0] = buf_x4(wr, voff | dead, static_cast<uint32_t>(kb) * 64);
   r.code = buf_u8(sr, coff | dead, static_cast<uint32_t>(kb) * 4);
 }
@@ -130,9 +130,9 @@ __device__ __forceinline__ void dequant(const RawA<FMT>& r, bf16x8 (&a)[4]) {
 }
 
 // Registers of one K block in flight: NMAT weight tiles and NCH activation chunks.
-template <int FMT, int NMAT, int NCH>
+template <int NMAT, int NCH>
 struct KStage {
-  RawA<FMT> w[NMAT];
+  RawA<FMT_MXFP4> w[NMAT];
   u32x4 b[NCH][4];
 };
 
@@ -150,25 +150,24 @@ struct WTiles {
   uint32_t soff[NMAT];
 };
 
-template <int FMT, int NMAT, int NCH>
-__device__ __forceinline__ void load_stage(KStage<FMT, NMAT, NCH>& st, const WTiles<NMAT>& wt,
-                                           __amdgpu_buffer_rsrc_t br, const uint32_t (&bvoff)[NCH], int kb,
-                                           uint32_t dead) {
+template <int NMAT, int NCH>
+__device__ __forceinline__ void load_stage(KStage<NMAT, NCH>& st, const WTiles<NMAT>& wt, __amdgpu_buffer_rsrc_t br,
+                                           const uint32_t (&bvoff)[NCH], int kb, uint32_t dead) {
 #pragma unroll
-  for (int m = 0; m < NMAT; ++m) load_raw<FMT>(wt.wr, wt.sr, wt.wvoff[m], wt.soff[m], kb, dead, st.w[m]);
+  for (int m = 0; m < NMAT; ++m) load_raw(wt.wr, wt.sr, wt.wvoff[m], wt.soff[m], kb, dead, st.w[m]);
   const uint32_t so = static_cast<uint32_t>(kb) * 256;
 #pragma unroll
   for (int c = 0; c < NCH; ++c)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) st.b[c][j] = buf_x4(br, (bvoff[c] | dead) + b_piece_bytes<FMT>(j), so);
+    for (int j = 0; j < 4; ++j) st.b[c][j] = buf_x4(br, (bvoff[c] | dead) + b_piece_bytes<FMT_MXFP4>(j), so);
 }
 
-template <int FMT, int NMAT, int NCH>
-__device__ __forceinline__ void compute_stage(const KStage<FMT, NMAT, NCH>& st, f32x4 (&acc)[NMAT][NCH]) {
+template <int NMAT, int NCH>
+__device__ __forceinline__ void compute_stage(const KStage<NMAT, NCH>& st, f32x4 (&acc)[NMAT][NCH]) {
 #pragma unroll
   for (int m = 0; m < NMAT; ++m) {
     bf16x8 a[4];
-    dequant<FMT>(st.w[m], a);
+    dequant<FMT_MXFP4>(st.w[m], a);
 #pragma unroll
     for (int c = 0; c < NCH; ++c)
 #pragma unroll
@@ -181,10 +180,9 @@ __device__ __forceinline__ void compute_stage(const KStage<FMT, NMAT, NCH>& st, 
 // K stages kept in flight: as many as fit next to the accumulators in the
 // 256 registers of occupancy 2 (a stage holds NMAT weight tiles, their scales
 // and NCH activation chunks), between 2 and 4.
-template <int FMT, int NMAT, int NCH>
+template <int NMAT, int NCH>
 constexpr int pipeline_depth() {
-  constexpr int wregs = 4;
-  constexpr int per_stage = NMAT * (wregs + 1) + NCH * 16;
+  constexpr int per_stage = NMAT * (4 + 1) + NCH * 16;
   constexpr int fit = (200 - NMAT * NCH * 4 - 24) / per_stage;
   return fit < 2 ? 2 : fit > 4 ? 4 : fit;
 }
@@ -194,10 +192,10 @@ constexpr int pipeline_depth() {
 // S register stages: the loads of the next S-1 K blocks are in flight while one
 // is computed.  Every step issues its loads (dead ones read zeros), so the
 // hardware counters wait for exactly the stage about to be used.
-template <int FMT, int NMAT, int NCH, int KS>
+template <int NMAT, int NCH, int KS>
 __device__ __forceinline__ void gemv_tile(const WTiles<NMAT>& wt, int K, int kw, __amdgpu_buffer_rsrc_t br,
                                           const uint32_t (&bvoff)[NCH], f32x4 (&acc)[NMAT][NCH]) {
-  constexpr int S = pipeline_depth<FMT, NMAT, NCH>();
+  constexpr int S = pipeline_depth<NMAT, NCH>();
   const int nkb = K / 128;
   const int kb_lo = kw * nkb / KS, kb_hi = (kw + 1) * nkb / KS;
   const int n = kb_hi - kb_lo;
@@ -206,7 +204,7 @@ __device__ __forceinline__ void gemv_tile(const WTiles<NMAT>& wt, int K, int kw,
   for (int m = 0; m < NMAT; ++m)
 #pragma unroll
     for (int c = 0; c < NCH; ++c) acc[m][c] = zero;
-  KStage<FMT, NMAT, NCH> st[S];
+  KStage<NMAT, NCH> st[S];
 #pragma unroll
   for (int s = 0; s < S - 1; ++s) load_stage(st[s], wt, br, bvoff, kb_lo + s, s < n ? 0u : kOutOfRange);
   // whole groups of S steps: loads and computes unconditional
@@ -239,7 +237,7 @@ __device__ __forceinline__ void gemv_tile(const WTiles<NMAT>& wt, int K, int kw,
 // each fetches complete lines, which lets the weights use the nontemporal policy
 // (measured on MI355X: 7.1 TB/s against 6.2 TB/s for the default policy on a
 // plain stream; bf16 experts, register loads -> LDS, H 2048, I 768, 128 experts,
-// top-8: 4 tokens 71.7 -> 61.4 us, 24 196 -> 170, 64 233 -> 201, 256 318 -> 227;
+// top-8: 4 tokens 71.7 -> 61.2 us, 24 188 -> 161, 256 318 -> 209;
 // a bf16 shared expert beside MXFP4 at 64 tokens, H 5120, 247 -> 235).
 // A K step covers 128 bytes of every row: one K block of FP8, two of MXFP4, half
 // a block of bf16.  Each wave owns a ring of stages in LDS (dma_depth); a stage
@@ -488,7 +486,7 @@ constexpr int dma_ring_bytes() {  // per wave, the larger of the NCH variants (W
          NMAT * kTileBytes;
 }
 
-// Counterpart of gemv_tile for FP8 and MXFP4: the same K range and
+// Counterpart of gemv_tile for every format: the same K range and
 // accumulation order, the weights through the wave's LDS ring of S stages (the
 // DMA of the next S-1 steps is in flight while one is computed; a dead step
 // still issues, reading zeros, so every step's wait count is exact).
@@ -901,65 +899,65 @@ __device__ __forceinline__ void decode_pass(const DecodeArgs& a, const BankView&
       wt.soff[m] = static_cast<uint32_t>(tile_row / 128) * (K / 128) * 4;
   }
   f32x4 acc[NMAT][NCH];
-  // FP8 always, MXFP4 when a K step (two K blocks) divides K: the LDS path
+  // the LDS path, except for MXFP4 where a K step (two K blocks) does not divide K
   if (K % dma_kstep<FMT>() == 0) {
-    {
-      DmaTiles<NMAT> dt;
-      dt.wr = wt.wr;
-      dt.sr = wt.sr;
-      const int dr = lane >> 3, dc = (lane & 7) ^ dr;  // DMA lane: row dr of 8, stored at slot lane & 7
+    DmaTiles<NMAT> dt;
+    dt.wr = wt.wr;
+    dt.sr = wt.sr;
+    const int dr = lane >> 3, dc = (lane & 7) ^ dr;  // DMA lane: row dr of 8, stored at slot lane & 7
 #pragma unroll
-      for (int m = 0; m < NMAT; ++m) {
-        const int tile_row = (STAGE == 0 && m >= RT) ? inter + wrow0 + 16 * (m - RT) : wrow0 + 16 * m;
+    for (int m = 0; m < NMAT; ++m) {
+      const int tile_row = (STAGE == 0 && m >= RT) ? inter + wrow0 + 16 * (m - RT) : wrow0 + 16 * m;
 #pragma unroll
-        for (int h = 0; h < 2; ++h) dt.voff[m][h] = static_cast<uint32_t>(tile_row + 8 * h + dr) * rb + dc * 16;
-        dt.soff[m] = FMT == FMT_MXFP4 ? static_cast<uint32_t>(tile_row + r16) * (K / 32) : wt.soff[m];
-      }
-      uint8_t* ring = smem + wave * dma_ring_bytes<FMT, NMAT, WIDE>();
-      if constexpr (KS == 1) {
-        // activation copies: copy v of chunk c of this wave covers columns
-        // q * (1024 / CB) + lane / (CB / 16), q = wave * act_copies + v
-        constexpr int CB = act_col_bytes<FMT>();
-        uint32_t avoff[NCH][act_copies<FMT>()];
+      for (int h = 0; h < 2; ++h) dt.voff[m][h] = static_cast<uint32_t>(tile_row + 8 * h + dr) * rb + dc * 16;
+      dt.soff[m] = FMT == FMT_MXFP4 ? static_cast<uint32_t>(tile_row + r16) * (K / 32) : wt.soff[m];
+    }
+    uint8_t* ring = smem + wave * dma_ring_bytes<FMT, NMAT, WIDE>();
+    if constexpr (KS == 1) {
+      // activation copies: copy v of chunk c of this wave covers columns
+      // q * (1024 / CB) + lane / (CB / 16), q = wave * act_copies + v
+      constexpr int CB = act_col_bytes<FMT>();
+      uint32_t avoff[NCH][act_copies<FMT>()];
 #pragma unroll
-        for (int c = 0; c < NCH; ++c)
+      for (int c = 0; c < NCH; ++c)
 #pragma unroll
-          for (int v = 0; v < act_copies<FMT>(); ++v) {
-            // (bf16: copy q of the step covers 8 columns of chunk q / 2)
-            const int q = FMT == FMT_BF16 ? (NCH == 1 ? wave & 1 : wave) : wave * act_copies<FMT>() + v;
-            const int colc = (FMT == FMT_BF16 ? q & 1 : q) * (1024 / CB) + lane / (CB / 16);
-            const int piece = act_piece_pos<FMT>(lane % (CB / 16), colc);
-            const int col = base + (FMT == FMT_BF16 ? q >> 1 : c) * 16 + colc;
-            if (col < sv.count) {
-              int row;
-              if (STAGE == 0) row = sv.shared ? sv.start + col : a.sorted[sv.start + col] / a.k;
-              else row = sv.shared ? a.M * a.k + sv.start + col : a.sorted[sv.start + col];
-              avoff[c][v] = static_cast<uint32_t>(row) * bstride * 2 + piece * 16;
-            } else {
-              avoff[c][v] = kOutOfRange;
-            }
+        for (int v = 0; v < act_copies<FMT>(); ++v) {
+          // (bf16: copy q of the step covers 8 columns of chunk q / 2)
+          const int q = FMT == FMT_BF16 ? (NCH == 1 ? wave & 1 : wave) : wave * act_copies<FMT>() + v;
+          const int colc = (FMT == FMT_BF16 ? q & 1 : q) * (1024 / CB) + lane / (CB / 16);
+          const int piece = act_piece_pos<FMT>(lane % (CB / 16), colc);
+          const int col = base + (FMT == FMT_BF16 ? q >> 1 : c) * 16 + colc;
+          if (col < sv.count) {
+            int row;
+            if (STAGE == 0) row = sv.shared ? sv.start + col : a.sorted[sv.start + col] / a.k;
+            else row = sv.shared ? a.M * a.k + sv.start + col : a.sorted[sv.start + col];
+            avoff[c][v] = static_cast<uint32_t>(row) * bstride * 2 + piece * 16;
+          } else {
+            avoff[c][v] = kOutOfRange;
           }
-        if constexpr (FMT == FMT_MXFP4) {
-          if (K <= kCodeRegSteps * dma_kstep<FMT>())
-            gemv_tile_dma_sh<FMT, NMAT, NCH, WIDE, true>(dt, K, wave, br, avoff, ring, aring, acc);
-          else
-            gemv_tile_dma_sh<FMT, NMAT, NCH, WIDE>(dt, K, wave, br, avoff, ring, aring, acc);
-        } else {
-          gemv_tile_dma_sh<FMT, NMAT, NCH, WIDE, false, CW>(dt, K, wave, br, avoff, ring, aring, acc);
         }
+      if constexpr (FMT == FMT_MXFP4) {
+        if (K <= kCodeRegSteps * dma_kstep<FMT>())
+          gemv_tile_dma_sh<FMT, NMAT, NCH, WIDE, true>(dt, K, wave, br, avoff, ring, aring, acc);
+        else
+          gemv_tile_dma_sh<FMT, NMAT, NCH, WIDE>(dt, K, wave, br, avoff, ring, aring, acc);
       } else {
-        if constexpr (FMT == FMT_MXFP4 && KS == kDecWaves && STAGE == 0) {
-          // aring: the code table's LDS, behind the waves' rings
-          if (code_table_fits<NMAT>(K)) gemv_tile_dma<FMT, NMAT, NCH, KS, true>(dt, K, kw, br, bvoff, ring, acc, aring, wrow0, inter);
-          else gemv_tile_dma<FMT, NMAT, NCH, KS>(dt, K, kw, br, bvoff, ring, acc);
-        } else {
-          gemv_tile_dma<FMT, NMAT, NCH, KS, false, CW>(dt, K, kw, br, bvoff, ring, acc);
-        }
+        gemv_tile_dma_sh<FMT, NMAT, NCH, WIDE, false, CW>(dt, K, wave, br, avoff, ring, aring, acc);
+      }
+    } else {
+      if constexpr (FMT == FMT_MXFP4 && KS == kDecWaves && STAGE == 0) {
+        // aring: the code table's LDS, behind the waves' rings
+        if (code_table_fits<NMAT>(K))
+          gemv_tile_dma<FMT, NMAT, NCH, KS, true>(dt, K, kw, br, bvoff, ring, acc, aring, wrow0, inter);
+        else
+          gemv_tile_dma<FMT, NMAT, NCH, KS>(dt, K, kw, br, bvoff, ring, acc);
+      } else {
+        gemv_tile_dma<FMT, NMAT, NCH, KS, false, CW>(dt, K, kw, br, bvoff, ring, acc);
       }
     }
   } else {
     if constexpr (FMT == FMT_MXFP4)  // the others' steps divide every K (a multiple of 128)
-      gemv_tile<FMT, NMAT, NCH, KS>(wt, K, kw, br, bvoff, acc);
+      gemv_tile<NMAT, NCH, KS>(wt, K, kw, br, bvoff, acc);
   }
 
   if constexpr (KS == 1) {
@@ -1047,7 +1045,8 @@ struct StageSmem {
       (FMT_R == FMT_FP8 || FMT_S == FMT_FP8) ? dma_ring_bytes<FMT_FP8, kNmat, WIDE && KS == 1>() : 0;
   static constexpr int kRingF4 =
       (FMT_R == FMT_MXFP4 || FMT_S == FMT_MXFP4) ? dma_ring_bytes<FMT_MXFP4, kNmat>() : 0;
-  static constexpr int kRingBf = (FMT_R == FMT_BF16 || FMT_S == FMT_BF16) ? dma_ring_bytes<FMT_BF16, kNmat, WIDE && KS == 1>() : 0;
+  static constexpr int kRingBf =
+      (FMT_R == FMT_BF16 || FMT_S == FMT_BF16) ? dma_ring_bytes<FMT_BF16, kNmat, WIDE && KS == 1>() : 0;
   static constexpr int kRingQ = kRingF8 > kRingF4 ? kRingF8 : kRingF4;
   static constexpr int kRing = kDecWaves * (kRingQ > kRingBf ? kRingQ : kRingBf);
   // without a K split the activation ring shared by the waves follows the waves' weight rings

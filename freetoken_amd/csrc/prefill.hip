@@ -368,7 +368,7 @@ __global__ void __launch_bounds__(kPThreads) prefill_gemm_kernel(PrefillGemmArgs
 // Gate/up: row group rg owns gate rows n0+32rg+[0,32) and up rows
 // I+n0+32rg+[0,32), so SwiGLU pairs registers; a workgroup covers 128
 // intermediate features.  Down: rows at or past N (the last tile when
-// N % 256 != 0) are read clamped to row N-1 and never stored.  The epilogues
+// N % 256 != 0) read zeros and are never stored.  The epilogues
 // are VALU work with the matrix cores idle: the gate/up epilogue quantises
 // without a division instruction (quant.h) and the down epilogue stores its
 // outputs as whole 128-byte rows through LDS.
@@ -568,7 +568,7 @@ __device__ __forceinline__ int swz64(int line) { return (line >> 1) & 3; }
 
 // Position of a running count in a ring of N.  (Unsigned: the signed remainders
 // were a dozen more scalar operations at the head of every step, before its
-// first LDS read: FP8 1-13 tiles a workgroup 0.3-0.8% of the call.)
+// first LDS read; FP8 calls gained 0.3-0.8%.)
 template <int N>
 __device__ __forceinline__ int ring(int i) {
   return static_cast<int>(static_cast<unsigned>(i) % N);
@@ -607,7 +607,8 @@ __global__ void __launch_bounds__(kQThreads) prefill_qgemm_kernel(PrefillGemmArg
   const uint32_t rb = FMT == FMT_BF16 ? 2u * K : FMT == FMT_FP8 ? 1u * K : static_cast<uint32_t>(K) / 2;
   const uint32_t xb = FMT == FMT_BF16 ? 2u * K : 1u * K;
 
-  for (int e = tid; e <= a.num_experts; e += kQThreads) s_blk[e] = static_cast<typename L::Blk>(a.cum[e] / BM);  // (published with the first routes)
+  // (published with the first tile's routes)
+  for (int e = tid; e <= a.num_experts; e += kQThreads) s_blk[e] = static_cast<typename L::Blk>(a.cum[e] / BM);
   int v = blockIdx.x;
   QTile cur;
   constexpr int kChunk = q_chunk<FMT, GATE_UP, BM>();
@@ -653,7 +654,8 @@ __global__ void __launch_bounds__(kQThreads) prefill_qgemm_kernel(PrefillGemmArg
   // relative to the tile), the next BM/64 waves 64 activation-scale columns each
   // (sbase, srange: the array this wave copies from; slanes lanes take part)
   const int slanes = wave < 4 ? (FMT == FMT_FP8 ? 4 : kWave) : wave < 4 + BM / 64 ? kWave : 0;
-  const int sdst = __builtin_amdgcn_readfirstlane(wave < 4 ? wave * (L::kWS / 4) : L::kWS + (wave - 4) * (L::kXS / (BM / 64)));
+  const int sdst = __builtin_amdgcn_readfirstlane(wave < 4 ? wave * (L::kWS / 4)
+                                                           : L::kWS + (wave - 4) * (L::kXS / (BM / 64)));
   uint64_t sbase = reinterpret_cast<uint64_t>(a.xs);
   uint32_t srange = kQuant ? static_cast<uint32_t>(xrows) * xsb : 0u;
   uint32_t svoff = 0;
@@ -713,7 +715,8 @@ __global__ void __launch_bounds__(kQThreads) prefill_qgemm_kernel(PrefillGemmArg
   auto issue_piece = [&](int q, int kb, int stg) {
     uint8_t* st = q_lds + stg * L::kStage;
     if (q < L::kACopies) {
-      lds_buf16(make_rsrc(reinterpret_cast<const void*>(wbase), wrange), st + (wave * L::kACopies + q) * 1024, avoff[q], static_cast<uint32_t>(kb) * L::kALine);
+      lds_buf16(make_rsrc(reinterpret_cast<const void*>(wbase), wrange), st + (wave * L::kACopies + q) * 1024,
+                avoff[q], static_cast<uint32_t>(kb) * L::kALine);
     } else {
       const int c = q - L::kACopies;
       lds_buf16(rsrc_x, st + L::kA + (wave * L::kBCopies + c) * 1024, xvoff[c], static_cast<uint32_t>(kb) * 128);
@@ -748,11 +751,12 @@ __global__ void __launch_bounds__(kQThreads) prefill_qgemm_kernel(PrefillGemmArg
   f32x4 acc[4][NCT];
 
   // K step kb from stage stg, scales from the groups that start at gb.  With
-  // ikb >= 0 the copies of step ikb into stage istg (groups from igb) are issued a few per column tile in the first tiles, between the
-  // LDS reads and MFMAs, instead of as one burst before the step (a burst
-  // stalls the wave's in-order issue until the memory pipeline takes it:
-  // measured 3% of the FP8 gate_up GEMM; MXFP4 with 256-route tiles, whose
-  // 3-stage ring already spills a few registers, keeps the burst).
+  // ikb >= 0 the copies of step ikb into stage istg (groups from igb) are issued
+  // a few per column tile in the first tiles, between the LDS reads and MFMAs,
+  // instead of as one burst before the step (a burst stalls the wave's in-order
+  // issue until the memory pipeline takes it: measured 3% of the FP8 gate_up
+  // GEMM; MXFP4 with 256-route tiles, which has no registers to spare, keeps the
+  // burst).
   constexpr bool kSpread = FMT != FMT_MXFP4 || BM < 256;
   constexpr int kPer = NCT == 8 ? 2 : (kPieces + NCT - 1) / NCT;  // pieces per column tile
   auto compute = [&](int kb, int stg, int gb, int ikb, int istg, int igb) {
@@ -953,7 +957,8 @@ __global__ void __launch_bounds__(kQThreads) prefill_qgemm_kernel(PrefillGemmArg
           if constexpr (!kQuant) {
             const int route = s_route[b][(BM / 2) * ch + 16 * i + r16];
             if (route < lim_col) {
-              uint16_t* const dst = a.out + static_cast<size_t>(t.shared ? a.numel + route : route) * a.inter + n0 + 32 * rg + g * 4;
+              const size_t arow = t.shared ? a.numel + route : route;
+              uint16_t* const dst = a.out + arow * a.inter + n0 + 32 * rg + g * 4;
               *reinterpret_cast<uint2*>(dst) = uint2{pk[0][0][0], pk[0][0][1]};
               *reinterpret_cast<uint2*>(dst + 16) = uint2{pk[0][1][0], pk[0][1][1]};
             }
