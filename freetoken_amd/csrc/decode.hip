@@ -237,8 +237,8 @@ __device__ __forceinline__ void gemv_tile(const WTiles<NMAT>& wt, int K, int kw,
 // each fetches complete lines, which lets the weights use the nontemporal policy
 // (measured on MI355X: 7.1 TB/s against 6.2 TB/s for the default policy on a
 // plain stream; bf16 experts, register loads -> LDS, H 2048, I 768, 128 experts,
-// top-8: 4 tokens 71.7 -> 61.2 us, 24 188 -> 161, 256 318 -> 209;
-// a bf16 shared expert beside MXFP4 at 64 tokens, H 5120, 247 -> 235).
+// top-8: 4 tokens 64.3 -> 58.7 us, 24 191 -> 162, 64 231 -> 198, 256 312 -> 221; a
+// bf16 shared expert beside 32 MXFP4 ones at 64 tokens, H 5120, I 1536, 150 -> 139).
 // A K step covers 128 bytes of every row: one K block of FP8, two of MXFP4, half
 // a block of bf16.  Each wave owns a ring of stages in LDS (dma_depth); a stage
 // holds NMAT tiles of 16 rows x 128 bytes.  Chunk c (16 bytes) of tile row r
@@ -1379,8 +1379,9 @@ static hipError_t launch_stage_t(int stage, const DecodeArgs& a, bool has_shared
     // 72.5-72.8 -> 69.6-70.6 us, b=2 115.4-116.1 -> 109.7-109.8 us; b=4
     // 160.1 -> 156.7 and 176.9 -> 175.7 us on two boxes, b=3 equal; up to 8
     // tokens C2 b=8 was 5% slower; MXFP4 at C3 b=1 0.8 us slower, so it
-    // keeps RT = 2; bf16 H 1024, I 512, 16 experts, top-2: 4 tokens 24.1 ->
-    // 22.7 us, H 4096, I 1536, 32 experts, top-8: 4 tokens 140.6 -> 138.5)
+    // keeps RT = 2; bf16 graph replays, H 1024, I 512, 16 experts, top-2: 4
+    // tokens 23.5 -> 22.0 us, 1 token 20.3 -> 19.4; H 4096, I 1536, 32 experts,
+    // top-8: 4 tokens 151 -> 147; H 2048, I 768, 128 experts equal)
     if ((FR == FMT_FP8 || FR == FMT_BF16) &&
         (a.M <= 4 ||
          static_cast<long long>(g2.x) * g2.y <= static_cast<long long>(cu_count()) * resident_per_cu<k2>()))
@@ -1402,8 +1403,8 @@ static hipError_t launch_stage_t(int stage, const DecodeArgs& a, bool has_shared
   if (heavy_shared && a.M <= 2) return launch_one<k1>(g1, a, stream);
   // one FP8 or bf16 token: K split two ways (half the rows per workgroup's row group
   // walk, twice the workgroups); interleaved A/B: C4 b=1 69.6 -> 68.9 us, C2
-  // b=1 30.2 -> 29.3 us; bf16 H 2048, I 768 32.3 -> 30.7, H 1024, I 512 22.8 ->
-  // 20.6; from two tokens equal or slower
+  // b=1 30.2 -> 29.3 us; bf16 H 2048, I 768, 128 experts 31.3 -> 29.4, H 1024, I
+  // 512, 16 experts 19.9 -> 19.4; from two tokens equal or slower
   if ((FR == FMT_FP8 || FR == FMT_BF16) && a.M == 1) {
     constexpr auto kh = decode_stage_kernel<FR, FS, 1, 2, 2>;
     return launch_one<kh>(dim3(a.H / 64, gy), a, stream);
